@@ -187,6 +187,12 @@ int i8l_w8a8_mm_supported(int64_t M, int64_t N, int64_t K, const i8l_config* cfg
  * int8_linear/kernel.py:127-134, re-derived for MI355X). Host-only. */
 int i8l_default_config(int64_t M, int64_t N, int64_t K, i8l_config* cfg_out);
 
+/* The config a call without an explicit one launches, given the one planned for it in *cfg (a
+ * tuned entry with tuned != 0, else i8l_default_config's): from 129 tokens on, the macro tile with
+ * the least modelled time (a tuned macro tile is kept up to 512 tokens).  i8l_w8a8_mm and its
+ * variants apply it when their cfg is NULL.  Host-only; no counterpart in the reference. */
+int i8l_launch_config(int64_t M, int64_t N, int64_t K, int32_t tuned, i8l_config* cfg);
+
 /*
  * Fused add + RMSNorm + per-token int8 quantize, one row per token:
  *   x = f32(x) (+ f32(residual));  residual_out = cast(x)          (when residual != NULL)

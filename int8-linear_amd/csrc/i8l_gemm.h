@@ -431,5 +431,10 @@ hipError_t launch_dma(int idx, const i8l_config& c, const int8_t* a, int64_t lda
                       const int8_t* b, int64_t ldb, const Epi& e, int K, hipStream_t st);
 hipError_t launch_dmap(int idx, const i8l_config& c, const int8_t* a, int64_t lda,
                        const int8_t* b, int64_t ldb, const Epi& e, int K, hipStream_t st);
+// Phased prefill tiles (i8l_gemm_phased.hip): the config's `stages` is kPhasedStages.
+constexpr int kPhasedStages = 9;
+int phased_index(const i8l_config& c, int64_t K);
+hipError_t launch_phased(int idx, const i8l_config& c, const int8_t* a, int64_t lda,
+                         const int8_t* b, int64_t ldb, const Epi& e, int K, hipStream_t st);
 
 }  // namespace i8l

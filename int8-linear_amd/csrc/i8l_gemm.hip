@@ -177,9 +177,78 @@ void default_config(int64_t M, int64_t N, int64_t K, i8l_config* c) {
   }
 }
 
+// ------------------------------------------------------------------ the tile a call launches
+// A call without an explicit configuration plans one (a tuned entry, else default_config) and
+// launches what this makes of it: from 129 tokens on (33 where the plan is a macro tile already),
+// the macro tile with the least modelled time,
+//   fixed + rounds * (step * K + turn) us.
+// A tile's `rounds` is 0.7 times the whole rounds its tiles make over the compute units plus 0.3
+// times the exact ratio (a round of which a part is idle is as long, but the clock is higher); of
+// the 128x128 phased tile two fit a compute unit, and one alone takes 0.6 of their time.  The three
+// numbers of each tile are fitted to its times over 33 weight shapes (K 1024-28672, N 1024-57344)
+// at 33-5000 tokens on MI355X (rms error 5-15%).  There the pick takes 1.007x the fastest tile's
+// time on the geometric mean, and 1.006x over eight of the shapes left out of the fit, against
+// 1.08-1.13x for the plan; at tuned shapes between their buckets (512, 1024, 2048, 4096 tokens)
+// the plan takes 1.2-1.3x.  So a tuned macro tile is kept up to 512 tokens, where buckets lie 8-16
+// tokens apart (a decode tile only to 128: one token more doubles its row blocks).  The phased tiles (K a multiple of 256, from 512) beat the ring of their own size at all
+// of these points but two, so the larger rings serve the other K.
+static void launch_config(int64_t M, int64_t N, int64_t K, bool tuned, i8l_config* c) {
+  struct MacroTile {
+    int bm, bn, warps, stages, group_m;
+    float fixed, step, turn;   // us, us per 1000 bytes of K, us
+  };
+  static constexpr MacroTile kMacro[] = {
+      {256, 256, 4, kPhasedStages, 4, 0.0f, 10.75f, 9.87f},
+      {256, 192, 4, kPhasedStages, 4, 0.6f, 8.85f, 7.04f},
+      {256, 128, 4, kPhasedStages, 4, 2.05f, 6.74f, 2.9f},
+      {128, 256, 4, kPhasedStages, 8, 3.82f, 7.58f, 0.44f},
+      {128, 192, 4, kPhasedStages, 8, 4.14f, 6.15f, 0.73f},
+      {128, 128, 4, kPhasedStages, 8, 1.94f, 8.37f, 1.47f},
+      {64, 64, 4, 4 + kPipelined, 8, 4.19f, 1.92f, 0.01f},
+      {128, 64, 4, 4 + kPipelined, 8, 2.42f, 3.05f, 1.92f},
+      {64, 128, 4, 4 + kPipelined, 8, 2.89f, 3.33f, 1.6f},
+      {64, 256, 8, 3 + kPipelined, 8, 3.67f, 6.07f, 0.4f},
+      {128, 128, 4, 4 + kPipelined, 8, 3.07f, 4.73f, 2.72f},
+      {256, 128, 8, 3 + kPipelined, 8, 1.24f, 7.66f, 4.8f},
+      {128, 256, 8, 3 + kPipelined, 8, 3.0f, 8.19f, 2.94f},
+      {256, 192, 8, 2 + kPipelined, 4, 4.56f, 10.72f, 3.31f},
+      {256, 256, 8, 2 + kPipelined, 4, 2.21f, 13.15f, 4.96f}};
+  const bool macro = dmap_index(*c) >= 0 || phased_index(*c, K) >= 0;
+  if (K % 128 != 0 || N % 64 != 0 || (M <= 128 && !macro) ||
+      (tuned && M <= (macro ? 512 : 128)))
+    return;
+  const bool phased = K % 256 == 0 && K >= 512;
+  const int64_t cus = cu_count();
+  float best = -1.0f;
+  for (const auto& t : kMacro) {
+    const bool ph = t.stages == kPhasedStages;
+    if (N % t.bn != 0 || (phased ? !ph && t.bm * t.bn >= 128 * 128 && t.bm > 64 : ph)) continue;
+    const int64_t tiles = ((M + t.bm - 1) / t.bm) * (N / t.bn);
+    const bool two = ph && t.bm * t.bn == 128 * 128;
+    const int64_t slots = two ? 2 * cus : cus, rest = tiles % slots;
+    const float last = rest == 0 ? 0.0f : two && rest <= cus ? 0.6f : 1.0f;
+    const float rounds = 0.7f * ((float)(tiles / slots) + last) + 0.3f * (float)tiles / (float)slots;
+    const float us = t.fixed + rounds * (t.step * 1e-3f * (float)K + t.turn);
+    if (best < 0.0f || us < best) {
+      best = us;
+      *c = i8l_config{t.bm, t.bn, 128, t.warps, t.stages, t.group_m};
+    }
+  }
+}
+
 }  // namespace i8l
 
 using namespace i8l;
+
+extern "C" int i8l_launch_config(int64_t M, int64_t N, int64_t K, int32_t tuned,
+                                 i8l_config* cfg) {
+  if (!cfg) {
+    set_error("i8l_launch_config: cfg is NULL");
+    return I8L_INVALID_ARG;
+  }
+  launch_config(M, N, K, tuned != 0, cfg);
+  return I8L_OK;
+}
 
 extern "C" int i8l_default_config(int64_t M, int64_t N, int64_t K, i8l_config* cfg_out) {
   if (!cfg_out) {
@@ -202,7 +271,7 @@ extern "C" int i8l_w8a8_mm_supported(int64_t M, int64_t N, int64_t K, const i8l_
     return I8L_UNSUPPORTED;
   }
   if (!stream_ok(c) && staged_index(c) < 0 && dma_index(c) < 0 && dmap_index(c) < 0 &&
-      !wlds_ok(c, K) && !wldsp_ok(c, K) && !wlds_split_ok(c, K)) {
+      phased_index(c, K) < 0 && !wlds_ok(c, K) && !wldsp_ok(c, K) && !wlds_split_ok(c, K)) {
     set_error("config %dx%dx%d w%d s%d g%d is not built into this library", c.bm, c.bn,
               c.bk, c.warps, c.stages, c.group_m);
     return I8L_UNSUPPORTED;
@@ -260,10 +329,12 @@ int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t*
     }
   }
   i8l_config c;
-  if (cfg)
+  if (cfg) {
     c = *cfg;
-  else
+  } else {
     default_config(M, N, K, &c);
+    launch_config(M, N, K, false, &c);
+  }
   int st = i8l_w8a8_mm_supported(M, N, K, &c);
   if (st != I8L_OK) return st;
   if (M == 0 || N == 0) return I8L_OK;
@@ -307,7 +378,10 @@ int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t*
     }
   }
   hipError_t err;
-  if (!fast || (wlds && !small_strides)) {
+  // the phased schedule keeps in-tile offsets (256 rows of either operand) in 32 bits
+  const bool phased = c.stages == kPhasedStages;
+  const bool phased_strides = stride_am <= INT32_MAX / 256 && stride_bn <= INT32_MAX / 256;
+  if (!fast || (wlds && !small_strides) || (phased && !phased_strides)) {
     const int64_t tiles = ((N + 63) / 64) * ((M + 63) / 64);
     if (tiles > INT32_MAX) {
       set_error("%s: %lld x %lld is too large for the generic kernel", who, (long long)M,
@@ -326,6 +400,8 @@ int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t*
     err = launch_wldsp(c, a, stride_am, b, stride_bn, e, hs);
   } else if (wlds && c.stages == 3) {
     err = launch_wlds(c, a, stride_am, b, stride_bn, e, K, hs);
+  } else if (phased) {
+    err = launch_phased(phased_index(c, K), c, a, stride_am, b, stride_bn, e, (int)K, hs);
   } else if (c.stages == 2) {
     err = launch_staged(staged_index(c), c, a, stride_am, b, stride_bn, e, (int)K, hs);
   } else if (c.stages >= 2 + kPipelined) {

@@ -13,7 +13,7 @@
 //
 // Configuration choice follows kernel.choose_config (reference kernel.py:137-160): per
 // device, the tuned table's largest M bucket at or below M for "KxN", else the library's
-// default rule.  Python hands each device's table over once (set_table) before the first
+// default rule; i8l_launch_config then makes of it what is launched.  Python hands each device's table over once (set_table) before the first
 // fast call on that device.
 
 #include <torch/extension.h>
@@ -71,8 +71,8 @@ void set_table(int device, const std::vector<std::vector<int64_t>>& rows) {
 
 bool has_table(int device) { return g_tables.count(device) != 0; }
 
-// false when the device's table has not been handed over yet
-bool choose(int device, int64_t m, int64_t n, int64_t k, i8l_config* c) {
+// false when the device's table has not been handed over yet; *tuned: c is a table entry
+bool choose(int device, int64_t m, int64_t n, int64_t k, i8l_config* c, bool* tuned = nullptr) {
   auto dt = g_tables.find(device);
   if (dt == g_tables.end()) return false;
   auto st = dt->second.shapes.find(kn_key(k, n));
@@ -80,13 +80,14 @@ bool choose(int device, int64_t m, int64_t n, int64_t k, i8l_config* c) {
     auto it = st->second.upper_bound(m);  // first bucket above M
     if (it != st->second.begin()) {
       *c = std::prev(it)->second;
+      if (tuned) *tuned = true;
       return true;
     }
   }
   return i8l_default_config(m, n, k, c) == I8L_OK;
 }
 
-// The configuration the fast path launches (bm, bn, bk, warps, stages, group_m),
+// The configuration the fast path plans (bm, bn, bk, warps, stages, group_m),
 // or None before the device's table is handed over.
 py::object config_for(int device, int64_t m, int64_t n, int64_t k) {
   i8l_config c;
@@ -112,7 +113,9 @@ py::object mm(const at::Tensor& a, const at::Tensor& b, const at::Tensor& sa,
   const int64_t m = a.size(0), k = a.size(1), n = b.size(1);
   if (b.size(0) != k || b.device() != dev) return py::none();
   i8l_config c;
-  if (!choose(dev.index(), m, n, k, &c) || c.bn <= 0 || c.bk <= 0 || n % c.bn || k % c.bk)
+  bool tuned = false;
+  if (!choose(dev.index(), m, n, k, &c, &tuned) ||
+      i8l_launch_config(m, n, k, tuned ? 1 : 0, &c) != I8L_OK || c.bn <= 0 || c.bk <= 0 || n % c.bn || k % c.bk)
     return py::none();
   if (!plain_vector(sa, at::kFloat, dev) || !plain_vector(sb, at::kFloat, dev)) return py::none();
   if ((sa.numel() != 1 && sa.numel() != m) || (sb.numel() != 1 && sb.numel() != n))

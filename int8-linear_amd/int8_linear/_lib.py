@@ -30,7 +30,7 @@ class CConfig(ctypes.Structure):
                 ("group_m", _I32)]
 
 
-EXPORTS = ("i8l_w8a8_mm", "i8l_w8a8_mm_supported", "i8l_default_config",
+EXPORTS = ("i8l_w8a8_mm", "i8l_w8a8_mm_supported", "i8l_default_config", "i8l_launch_config",
            "i8l_add_rmsnorm_quant", "i8l_silu_mul_quant", "i8l_quant_per_token",
            "i8l_w8a8_mm_dynq", "i8l_w8a8_mm_dynq_supported",
            "i8l_silu_mul_quant_mm", "i8l_silu_mul_quant_mm_supported", "i8l_w8a8_mm_ws",
@@ -56,6 +56,7 @@ def lib() -> ctypes.CDLL:
                               _P, _I64, _I32, _I64, _I64, _I64, ctypes.POINTER(CConfig), _P]
     L.i8l_w8a8_mm_supported.argtypes = [_I64, _I64, _I64, ctypes.POINTER(CConfig)]
     L.i8l_default_config.argtypes = [_I64, _I64, _I64, ctypes.POINTER(CConfig)]
+    L.i8l_launch_config.argtypes = [_I64, _I64, _I64, _I32, ctypes.POINTER(CConfig)]
     L.i8l_add_rmsnorm_quant.argtypes = [_P, _P, _P, ctypes.c_float, _P, _P, _P, _I64, _I64, _I32,
                                         _I32, _I32, _P]
     L.i8l_silu_mul_quant.argtypes = [_P, _P, _P, _I64, _I64, _I32, _I32, _I32, _P]

@@ -54,7 +54,9 @@ class Config:
       3 <= stages <= 8, bm >= 128: a ring of `stages` LDS buffers filled by direct-to-LDS
         loads;
       stages >= 10: a ring of stages - 8 buffers (2 is a double buffer) with the LDS
-        fragment reads of each MFMA substep overlapped with the MFMAs of the one before.
+        fragment reads of each MFMA substep overlapped with the MFMAs of the one before;
+      stages == 9: the phased schedule (4 waves, persistent over the tiles, bk 128, K a
+        multiple of 256 from 512 on).
     A configuration the library was not built with raises NotSupported.
     """
 
@@ -129,6 +131,29 @@ def choose_config(m: int, n: int, k: int) -> Config:
     return cfg
 
 
+def launch_config(m: int, n: int, k: int, planned: Config | None = None) -> Config:
+    """The config a call without an explicit one launches (i8l_launch_config): choose_config's
+    (or `planned`, as a tuned one), and from 129 tokens on the macro tile with the least
+    modelled time where no tuned entry lies close below M."""
+    tuned = planned is not None or tuned_config(m, n, k) is not None
+    p = planned or choose_config(m, n, k)
+    c = _lib.CConfig(p.bm, p.bn, p.bk, p.warps, p.stages, p.group_m)
+    _lib.check(_lib.lib().i8l_launch_config(m, n, k, int(tuned), c), NotSupported)
+    return Config(c.bm, c.bn, c.bk, c.warps, c.stages, c.group_m)
+
+
+_launched: dict[tuple[int, int, int, int], Config] = {}
+
+
+def _auto_config(m: int, n: int, k: int) -> Config:
+    """launch_config, remembered per device and shape."""
+    key = (torch.cuda.current_device(), m, n, k)
+    cfg = _launched.get(key)
+    if cfg is None:
+        cfg = _launched[key] = launch_config(m, n, k)
+    return cfg
+
+
 def _table_rows(device: int) -> list[list[int]]:
     """This device's tuned table as rows (k, n, m, bm, bn, bk, warps, stages, group_m), for the
     C++ binding's configuration lookup."""
@@ -189,8 +214,8 @@ def w8a8_mm(
     scales and bias are ignored.  cached_launch is accepted for API compatibility; every
     launch is a direct C call already.
 
-    Without an explicit config the call goes through the C++ binding when it is built,
-    which chooses the same configuration (by the operands' device) and launches the same
+    Without an explicit config it is launch_config's, and the call goes through the C++ binding
+    when it is built, which chooses the same configuration (by the operands' device) and launches the same
     kernel; anything but the plain case comes back here.
     """
     if config is None and not raw:
@@ -208,7 +233,7 @@ def w8a8_mm(
     same_device(a_q.device, b_q=b_q, scale_a=scale_a, scale_b=scale_b, bias=bias)
     m, k = a_q.shape
     n = b_q.shape[1]
-    cfg = config or choose_config(m, n, k)
+    cfg = config or _auto_config(m, n, k)
     if n % cfg.bn or k % cfg.bk:
         raise NotSupported(f"N={n} and K={k} must divide the {cfg.name} tile")
     # Scales and bias are read as flat stride-1 arrays; contiguous() is free when they

@@ -63,6 +63,10 @@ DMAP_TILES = [(256, 256, 64, 8, 3), (256, 256, 64, 8, 4), (256, 256, 64, 8, 5),
               (256, 192, 128, 8, 2)]
 
 
+# (BM, BN) of the built phased tiles: 4 waves, 128-byte K steps (stages 9)
+PHASED = 9
+PHASED_TILES = [(256, 256), (256, 192), (256, 128), (128, 256), (128, 192), (128, 128)]
+
 # (MT, NC, KS, W) of the built persistent single-step decode tiles (stages 4): K = 64*KS*W
 WLDSP_TILES = [(1, 16, 2, 16), (2, 16, 2, 16), (1, 32, 2, 16), (1, 16, 4, 16),
                (1, 16, 4, 8), (2, 16, 4, 8), (4, 16, 4, 8), (1, 16, 8, 8),
@@ -146,6 +150,11 @@ def candidate_configs(m: int, k: int, n: int) -> list[Config]:
                 cfg = Config(bm, bn, bk, w, st + PIPELINED, g)
                 if supported(m, n, k, cfg):
                     out.append(cfg)
+        for bm, bn in PHASED_TILES:
+            for g in (4, 8):
+                cfg = Config(bm, bn, 128, 4, PHASED, g)
+                if supported(m, n, k, cfg):
+                    out.append(cfg)
     return out
 
 
@@ -198,7 +207,8 @@ def refine_candidates(m: int, k: int, n: int, stages=(3, 5)) -> list[Config]:
     from int8_linear.kernel import tuned_config
     cur = tuned_config(m, n, k) or default_config(m, n, k)
     # bn <= 64 at stages 3-5: wider tiles at those stages are prefill rings (gemm_dma)
-    new = [c for c in candidate_configs(m, k, n) if c.stages in stages and c.bn <= 64]
+    new = [c for c in candidate_configs(m, k, n)
+           if c.stages in stages and (c.bn <= 64 or c.stages == PHASED)]
     return [cur] + [c for c in new if c != cur]
 
 

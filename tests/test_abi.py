@@ -458,3 +458,28 @@ def test_tuner_candidate_sets(monkeypatch):
     assert not any(map(split, tune.candidate_configs(128, 4096, 28672)))
     assert tune.parse_ms("capture") == list(tune.CAPTURE_SIZES)
     assert tune.parse_ms("1,2,17") == [1, 2, 17]
+
+
+def test_launch_config_takes_every_planned_shape():
+    """What a call launches is built and takes the shape whatever was planned; up to 128 tokens a
+    decode plan is launched as it is, and so is a tuned macro tile up to 512; beyond, the pick does
+    not depend on the plan; shapes no macro tile divides keep their plan."""
+    def launched(m, n, k, plan=None, tuned=0):
+        p = plan or default_config(m, n, k)
+        c = _lib.CConfig(p.bm, p.bn, p.bk, p.warps, p.stages, p.group_m)
+        assert _lib.lib().i8l_launch_config(m, n, k, tuned, ctypes.byref(c)) == _lib.OK
+        return Config(c.bm, c.bn, c.bk, c.warps, c.stages, c.group_m)
+
+    for m in (1, 17, 32, 33, 64, 128, 129, 300, 512, 777, 1025, 4096, 16384):
+        for k in (64, 128, 256, 384, 512, 2048, 2112, 5120, 13824):
+            for n in (4, 48, 64, 192, 320, 2304, 5504, 57344):
+                c = launched(m, n, k)
+                assert kernel.supported(m, n, k, c), (m, n, k, c.name)
+                if m <= 128 and default_config(m, n, k).stages < 9 or k % 128 or n % 64:
+                    assert c == default_config(m, n, k), (m, n, k)
+    ring, decode = Config(64, 192, 128, 4, 12, 4), Config(32, 32, 128, 16, 3, 1)
+    assert launched(512, 6144, 4096, ring, 1) == ring
+    assert launched(128, 4096, 2048, decode, 1) == decode
+    assert launched(129, 4096, 2048, decode, 1) != decode
+    for plan in (ring, Config(256, 256, 128, 8, 10, 4), default_config(777, 6144, 4096)):
+        assert launched(777, 6144, 4096, plan, 1) == Config(128, 192, 128, 4, 9, 8)

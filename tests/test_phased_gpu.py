@@ -1,0 +1,95 @@
+"""The phased prefill tiles where they can go wrong: K from the least they take, an odd and an
+even number of step pairs, a ragged last row block, one token, several tiles a workgroup (the
+next tile's first steps requested in the last two of this one), every output and bias dtype and
+scale layout, bit for bit against the CPU oracle."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from helpers import bits, ints, np_, say
+from int8_linear import Config, kernel, tune, w8a8_mm
+from oracle import oracle as o
+
+pytestmark = pytest.mark.gpu
+
+TILES = [Config(bm, bn, 128, 4, tune.PHASED, 4) for bm, bn in tune.PHASED_TILES]
+ids = lambda c: c.name.replace(" ", "_")
+
+
+@pytest.mark.parametrize("config", TILES, ids=ids)
+@pytest.mark.parametrize("m,k", [(1, 512), (129, 768), (256, 1024), (511, 1280)])
+def test_int32_product_is_exact(config, m, k):
+    n = 3 * config.bn
+    say(f"phased raw {config.name} m={m} k={k} n={n}")
+    a, w = ints((m, k), m + k), ints((n, k), n)
+    one = torch.ones(1, device="cuda")
+    got = w8a8_mm(a, w.t(), one, one, raw=True, config=config)
+    assert np.array_equal(np_(got), o.gemm_i32(np_(a), np_(w)))
+
+
+@pytest.mark.parametrize("config", TILES, ids=ids)
+def test_several_tiles_a_workgroup(config):
+    """At least two tiles on every workgroup and a ragged third round, called three times."""
+    slots = 256 * (2 if config.bm * config.bn == 128 * 128 else 1)
+    m, k = 9 * config.bm - 5, 512
+    n = config.bn * (-(-(2 * slots + 7) // 9))
+    say(f"phased several tiles {config.name} m={m} k={k} n={n}")
+    a, w = ints((m, k), 3), ints((n, k), 4)
+    one = torch.ones(1, device="cuda")
+    ref = o.gemm_i32(np_(a), np_(w))
+    for _ in range(3):
+        got = w8a8_mm(a, w.t(), one, one, raw=True, config=config)
+        assert np.array_equal(np_(got), ref)
+
+
+@pytest.mark.parametrize("config", TILES, ids=ids)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+def test_every_bias_and_scale(config, dtype):
+    code = {torch.bfloat16: o.BF16, torch.float16: o.F16, torch.float32: o.F32}
+    m, k, n = 300, 512, 2 * config.bn
+    a, w = ints((m, k), 31), ints((n, k), 32)
+    acc = o.gemm_i32(np_(a), np_(w))
+    g = torch.Generator().manual_seed(33)
+    for per_row, per_col in ((True, True), (True, False), (False, True)):
+        sa = (torch.rand((m, 1) if per_row else (1,), generator=g) * 1e-2 + 1e-3).cuda()
+        sb = (torch.rand((n, 1) if per_col else (1,), generator=g) * 1e-2 + 1e-3).cuda()
+        for bd in (None, torch.bfloat16, torch.float16, torch.float32):
+            say(f"phased {config.name} {dtype} row={per_row} col={per_col} bias={bd}")
+            bias = torch.randn(n, generator=g).to(bd).cuda() if bd else None
+            got = w8a8_mm(a, w.t(), sa, sb, dtype, bias, config=config)
+            b = None if bd is None else np_(bias) if bd == torch.float32 else bits(bias)
+            ref = o.epilogue(acc, np_(sa), np_(sb), b, o.NONE if bd is None else code[bd],
+                             code[dtype])
+            out = np_(got) if dtype == torch.float32 else bits(got)
+            assert np.array_equal(out, ref), (per_row, per_col, bd)
+
+
+def test_wide_strides_take_the_generic_kernel():
+    """Row strides past what 32-bit in-tile offsets hold (256 rows) leave the phased kernel."""
+    config, m, k, n = TILES[0], 3, 512, 256
+    stride = (2 ** 31 - 1) // 256 + 1 + 15 & ~15
+    say(f"phased wide stride {stride}")
+    a, w = ints((m, k), 5), ints((n, k), 6)
+    wide = torch.zeros((m - 1) * stride + k, dtype=torch.int8, device="cuda")
+    view = wide.as_strided((m, k), (stride, 1))
+    view.copy_(a)
+    one = torch.ones(1, device="cuda")
+    got = w8a8_mm(view, w.t(), one, one, raw=True, config=config)
+    assert np.array_equal(np_(got), o.gemm_i32(np_(a), np_(w)))
+
+
+@pytest.mark.parametrize("m,k,n", [(129, 512, 640), (300, 2752, 5504), (777, 4096, 1536),
+                                   (640, 1920, 768), (200, 448, 320)])
+def test_launched_without_a_config(m, k, n):
+    """What a call without a configuration launches (the macro tile with the least modelled time, or
+    the plan where none divides the shape), against the oracle."""
+    say(f"launch_config m={m} k={k} n={n}: {kernel.launch_config(m, n, k).name}")
+    a, w = ints((m, k), m), ints((n, k), n)
+    sa = torch.rand((m, 1), generator=torch.Generator().manual_seed(1)).cuda() * 1e-2
+    sb = torch.rand((n, 1), generator=torch.Generator().manual_seed(2)).cuda() * 1e-2
+    got = w8a8_mm(a, w.t(), sa, sb)
+    ref = o.epilogue(o.gemm_i32(np_(a), np_(w)), np_(sa), np_(sb), None, o.NONE, o.BF16)
+    assert np.array_equal(bits(got), ref)
