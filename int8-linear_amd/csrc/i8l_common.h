@@ -118,6 +118,18 @@ __device__ __forceinline__ uint32_t code_rne(float v) {
   const float t = fminf(fmaxf(v, -128.0f), 127.0f) + 12582912.0f;
   return __float_as_uint(t) & 0xffu;
 }
+// The codes of four values as the bytes of a word, for the quantizer kernels: the clamp is one
+// v_med3_f32 (which like min(max(v, -128), 127) gives -128 for a NaN), and three byte permutes
+// take the place of the masks and shifts.  (The folded decode kernels gain nothing from it: the
+// 28-layer stand-in at one token 541 us either way.)
+__device__ __forceinline__ uint32_t code_rne_bits(float v) {
+  return __float_as_uint(__builtin_amdgcn_fmed3f(v, -128.0f, 127.0f) + 12582912.0f);
+}
+__device__ __forceinline__ uint32_t code_rne4(float a, float b, float c, float d) {
+  const uint32_t lo = __builtin_amdgcn_perm(code_rne_bits(b), code_rne_bits(a), 0x0c0c0400u);
+  const uint32_t hi = __builtin_amdgcn_perm(code_rne_bits(d), code_rne_bits(c), 0x0c0c0400u);
+  return __builtin_amdgcn_perm(hi, lo, 0x05040100u);
+}
 
 // exp(x) for float x, defined so that host and device give identical bits: Cody-Waite
 // range reduction x = k*ln2 + r (k = rne(x*log2(e)), ln2 split in a short head and a

@@ -197,6 +197,22 @@ def test_silu_mul_quant_every_bf16_gate(i, m):
             assert np.array_equal(np_(s), s0), np.argwhere(np_(s) != s0)[:5]
 
 
+@pytest.mark.parametrize("round_silu", [False, True])
+def test_silu_value_of_every_bf16_gate(round_silu):
+    """Each finite bf16 gate in a row of its own (times 1), whose scale is then |y| / 127: the
+    rounded value itself, which the codes of a mixed row show only to 1 in 127.  (Rounded, it comes
+    from the hardware's exp2 instead of the canonical one.)"""
+    say(f"silu_mul_quant the value of every bf16 gate round={round_silu}")
+    pats = np.arange(1 << 16, dtype=np.uint32)
+    pats = pats[((pats >> 7) & 0xff) != 255].astype(np.uint16)
+    gate = from_bits(np.repeat(pats[:, None], 8, axis=1), device="cpu")
+    gu = torch.cat([gate, torch.ones_like(gate)], dim=1).cuda()
+    q, s = fq.silu_mul_quant(gu, round_silu=round_silu)
+    q0, s0 = o.silu_mul_quant(bits(gu), o.BF16, round_silu, True)
+    bad = np.flatnonzero((np_(s) != s0).reshape(-1) | (np_(q) != q0).any(axis=1))[:5]
+    assert bad.size == 0, [(hex(pats[i]), float(np_(s)[i, 0]), float(s0.reshape(-1)[i])) for i in bad]
+
+
 @pytest.mark.parametrize("m", [1, 16, 128, 1024, 4096])
 def test_silu_mul_quant_config2(m):
     """BASELINE config 2 at full size: bit-exact against the oracle, and against the
