@@ -113,7 +113,7 @@ def _link_binding(obj: Path) -> Path:
     out = LIB.with_name("_i8l_fast" + sysconfig.get_config_var("EXT_SUFFIX"))
     tmp = out.with_suffix(".tmp")
     cmd = [CXX, "-shared", str(obj), *[f"-L{p}" for p in library_paths()], "-lc10",
-           "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python", f"-L{LIB.parent}",
+           "-lc10_hip", "-ltorch_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python", f"-L{LIB.parent}",
            "-lint8_linear_amd", "-Wl,-rpath,$ORIGIN", "-o", str(tmp)]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:

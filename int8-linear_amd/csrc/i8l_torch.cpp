@@ -17,6 +17,8 @@
 // fast call on that device.
 
 #include <torch/extension.h>
+#include <ATen/hip/EmptyTensor.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/hip/HIPStream.h>
 
 #include <algorithm>
@@ -95,6 +97,25 @@ py::object config_for(int device, int64_t m, int64_t n, int64_t k) {
   return py::make_tuple(c.bm, c.bn, c.bk, c.warps, c.stages, c.group_m);
 }
 
+// A fresh contiguous tensor on `like`'s device: at::empty's allocation (the caching allocator, under
+// a guard of the device) without its way through the dispatcher, which costs about as much again
+// on every output.  With a dispatch mode, a tracer or a function transform active, or a tensor
+// that is not a plain one, it goes through the dispatcher.
+at::Tensor empty_like_on(const at::Tensor& like, at::IntArrayRef size, at::ScalarType dtype) {
+  using c10::DispatchKey;
+  static constexpr c10::DispatchKeySet kWatched(
+      {DispatchKey::Python, DispatchKey::PythonTLSSnapshot, DispatchKey::PythonDispatcher,
+       DispatchKey::PreDispatch, DispatchKey::Functionalize, DispatchKey::FuncTorchBatched,
+       DispatchKey::FuncTorchBatchedDecomposition, DispatchKey::FuncTorchGradWrapper,
+       DispatchKey::FuncTorchDynamicLayerFrontMode, DispatchKey::FuncTorchDynamicLayerBackMode,
+       DispatchKey::FuncTorchVmapMode, DispatchKey::Batched, DispatchKey::VmapMode,
+       DispatchKey::TESTING_ONLY_GenericMode, DispatchKey::DeferredInit, DispatchKey::Fake,
+       DispatchKey::Tracer});
+  if ((c10::impl::tls_local_dispatch_key_set().included_ | like.key_set()).has_any(kWatched))
+    return at::empty(size, like.options().dtype(dtype));
+  return at::detail::empty_cuda(size, dtype, like.device(), std::nullopt);
+}
+
 // Launches made through this module (every entry point), for tests that check it was used.
 int64_t g_launches = 0;
 
@@ -132,12 +153,12 @@ py::object mm(const at::Tensor& a, const at::Tensor& b, const at::Tensor& sa,
       return py::none();
     bias_ptr = bt.data_ptr();
   }
-  at::Tensor out = at::empty({m, n}, a.options().dtype(out_dtype));
+  at::Tensor out = empty_like_on(a, {m, n}, out_dtype);
   // a split of K takes its int32 partial planes from the caching allocator (stream-ordered,
   // and from the graph's pool under capture)
   const int64_t ws_bytes = i8l_w8a8_mm_workspace_bytes(m, n, k, &c);
   at::Tensor ws;
-  if (ws_bytes > 0) ws = at::empty({ws_bytes}, a.options().dtype(at::kByte));
+  if (ws_bytes > 0) ws = empty_like_on(a, {ws_bytes}, at::kByte);
   const int st = i8l_w8a8_mm_ws(
       (const int8_t*)a.data_ptr(), a.stride(0), a.stride(1), (const int8_t*)b.data_ptr(),
       b.stride(0), b.stride(1), (const float*)sa.data_ptr(), sa.numel(),
@@ -164,10 +185,10 @@ py::object add_rmsnorm_quant(const at::Tensor& x, const c10::optional<at::Tensor
         r.device() != x.device())
       return py::none();
     rptr = r.data_ptr();
-    rout = at::empty_like(x);
+    rout = empty_like_on(x, x.sizes(), x.scalar_type());   // (x is contiguous)
   }
-  at::Tensor q = at::empty({M, H}, x.options().dtype(at::kChar));
-  at::Tensor s = at::empty({M, 1}, x.options().dtype(at::kFloat));
+  at::Tensor q = empty_like_on(x, {M, H}, at::kChar);
+  at::Tensor s = empty_like_on(x, {M, 1}, at::kFloat);
   if (M) {
     const int st = i8l_add_rmsnorm_quant(x.data_ptr(), rptr, w.data_ptr(), (float)eps,
                                          (int8_t*)q.data_ptr(), (float*)s.data_ptr(),
@@ -184,8 +205,8 @@ py::object silu_mul_quant(const at::Tensor& gu, bool precise_div, bool round_sil
   const int32_t act = act_code(gu.scalar_type());
   if (act < 0) return py::none();
   const int64_t M = gu.size(0), I = gu.size(1) / 2;
-  at::Tensor q = at::empty({M, I}, gu.options().dtype(at::kChar));
-  at::Tensor s = at::empty({M, 1}, gu.options().dtype(at::kFloat));
+  at::Tensor q = empty_like_on(gu, {M, I}, at::kChar);
+  at::Tensor s = empty_like_on(gu, {M, 1}, at::kFloat);
   if (M && I) {
     const int st = i8l_silu_mul_quant(gu.data_ptr(), (int8_t*)q.data_ptr(), (float*)s.data_ptr(),
                                       M, I, act, round_silu ? 1 : 0, precise_div ? 1 : 0,
@@ -202,8 +223,8 @@ py::object quant_per_token(const at::Tensor& x, bool precise_div) {
   if (x.stride(1) != 1 && H > 1) return py::none();
   const int32_t act = act_code(x.scalar_type());
   if (act < 0) return py::none();
-  at::Tensor q = at::empty({M, H}, x.options().dtype(at::kChar));
-  at::Tensor s = at::empty({M, 1}, x.options().dtype(at::kFloat));
+  at::Tensor q = empty_like_on(x, {M, H}, at::kChar);
+  at::Tensor s = empty_like_on(x, {M, 1}, at::kFloat);
   if (M && H) {
     const int64_t ldx = M > 1 ? x.stride(0) : H;
     const int st = i8l_quant_per_token(x.data_ptr(), ldx, (int8_t*)q.data_ptr(),

@@ -38,7 +38,7 @@ _ACT = {torch.bfloat16: _lib.BF16, torch.float16: _lib.F16}
 def _fast(name: str, *args):
     """The call through the C++ binding, or None (not built, or not the plain case: the
     Python path below then handles it, with its own checks and errors)."""
-    f = _lib.fast()
+    f = _lib._fast_mod or _lib.fast()
     if f is None:
         return None
     try:

@@ -168,7 +168,7 @@ def _table_rows(device: int) -> list[list[int]]:
 
 def _fast_mm(a_q, b_q, scale_a, scale_b, out_dtype, bias):
     """The launch through the C++ binding, or None (not built, or not the plain case)."""
-    f = _lib.fast()
+    f = _lib._fast_mod or _lib.fast()
     if f is None:
         return None
     try:

@@ -8,7 +8,7 @@ from __future__ import annotations
 import pytest
 import torch
 
-from helpers import ints, say
+from helpers import ints, randn, say
 from int8_linear import _lib, kernel
 from int8_linear import fused_quant as fq
 from int8_linear import vllm_patch
@@ -133,3 +133,27 @@ def test_vllm_entry_uses_the_binding_and_records_configs():
     assert vllm_patch.CALLS == calls + 1 and fast().launches() == before + 1
     assert vllm_patch.CONFIGS[(4, 2048, 2048)] == choose_config(4, 2048, 2048).name
     assert torch.equal(out, kernel.w8a8_mm(a, w.t(), sa, sb, config=choose_config(4, 2048, 2048)))
+
+
+def test_outputs_under_a_dispatch_mode():
+    """The binding allocates its outputs past the dispatcher, except where a dispatch mode or a
+    function transform is active: a mode then sees the allocations, and the outputs are the same."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    seen = []
+
+    class Watch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    say("binding outputs under a dispatch mode")
+    x = randn((5, 2048), 3)
+    q0, s0 = fq.quant_per_token(x)
+    before = fast().launches()
+    with Watch():
+        q, s = fq.quant_per_token(x)
+    assert fast().launches() == before + 1
+    assert sum("empty" in f for f in seen) == 2
+    assert torch.equal(q, q0) and torch.equal(s, s0)
+    assert q.is_contiguous() and not q.requires_grad and q.device == x.device
