@@ -386,7 +386,7 @@ int cu_count();   // compute units of the current device, 256 without one
 bool stream_ok(const i8l_config& c);
 bool wlds_ok(const i8l_config& c, int64_t K);
 bool wlds_split_ok(const i8l_config& c, int64_t K);
-int64_t wlds_split_workspace(const i8l_config& c, int64_t M, int64_t N);
+int64_t split_workspace(const i8l_config& c, int64_t M, int64_t N, int64_t K);   // 0: no split
 hipError_t launch_wlds_split(const i8l_config& c, const int8_t* a, int64_t lda,
                              const int8_t* b, int64_t ldb, const Epi& e, int64_t K,
                              int32_t* ws, hipStream_t st);
@@ -431,6 +431,15 @@ hipError_t launch_dma(int idx, const i8l_config& c, const int8_t* a, int64_t lda
                       const int8_t* b, int64_t ldb, const Epi& e, int K, hipStream_t st);
 hipError_t launch_dmap(int idx, const i8l_config& c, const int8_t* a, int64_t lda,
                        const int8_t* b, int64_t ldb, const Epi& e, int K, hipStream_t st);
+// Shared-ring tiles (i8l_gemm_ring.hip): the config's `stages` is kRingStages and `bn` 64, and
+// group_m > 1 splits K as stages 5 does.  A ring takes as many slots as fit the LDS.
+constexpr int kRingStages = 6;
+__host__ __device__ constexpr int ring_slots(int mt) {
+  return 160 * 1024 / ((64 + 16 * mt) * 128);
+}
+bool ring_ok(const i8l_config& c, int64_t K);
+hipError_t launch_ring(const i8l_config& c, const int8_t* a, int64_t lda, const int8_t* b,
+                       int64_t ldb, const Epi& e, int64_t K, hipStream_t st);
 // Phased prefill tiles (i8l_gemm_phased.hip): the config's `stages` is kPhasedStages.
 constexpr int kPhasedStages = 9;
 int phased_index(const i8l_config& c, int64_t K);

@@ -179,60 +179,96 @@ void default_config(int64_t M, int64_t N, int64_t K, i8l_config* c) {
 
 // ------------------------------------------------------------------ the tile a call launches
 // A call without an explicit configuration plans one (a tuned entry, else default_config) and
-// launches what this makes of it: from 129 tokens on (33 where the plan is a macro tile already),
-// the macro tile with the least modelled time,
+// launches what this makes of it: the tile with the least modelled time,
 //   fixed + rounds * (step * K + turn) us.
-// A tile's `rounds` is 0.7 times the whole rounds its tiles make over the compute units plus 0.3
-// times the exact ratio (a round of which a part is idle is as long, but the clock is higher); of
-// the 128x128 phased tile two fit a compute unit, and one alone takes 0.6 of their time.  The three
-// numbers of each tile are fitted to its times over 33 weight shapes (K 1024-28672, N 1024-57344)
-// at 33-5000 tokens on MI355X (rms error 5-15%).  There the pick takes 1.007x the fastest tile's
-// time on the geometric mean, and 1.006x over eight of the shapes left out of the fit, against
-// 1.08-1.13x for the plan; at tuned shapes between their buckets (512, 1024, 2048, 4096 tokens)
-// the plan takes 1.2-1.3x.  So a tuned macro tile is kept up to 512 tokens, where buckets lie 8-16
-// tokens apart (a decode tile only to 128: one token more doubles its row blocks).  The phased tiles (K a multiple of 256, from 512) beat the ring of their own size at all
-// of these points but two, so the larger rings serve the other K.
-static void launch_config(int64_t M, int64_t N, int64_t K, bool tuned, i8l_config* c) {
-  struct MacroTile {
-    int bm, bn, warps, stages, group_m;
-    float fixed, step, turn;   // us, us per 1000 bytes of K, us
-  };
-  static constexpr MacroTile kMacro[] = {
-      {256, 256, 4, kPhasedStages, 4, 0.0f, 10.75f, 9.87f},
-      {256, 192, 4, kPhasedStages, 4, 0.6f, 8.85f, 7.04f},
-      {256, 128, 4, kPhasedStages, 4, 2.05f, 6.74f, 2.9f},
-      {128, 256, 4, kPhasedStages, 8, 3.82f, 7.58f, 0.44f},
-      {128, 192, 4, kPhasedStages, 8, 4.14f, 6.15f, 0.73f},
-      {128, 128, 4, kPhasedStages, 8, 1.94f, 8.37f, 1.47f},
-      {64, 64, 4, 4 + kPipelined, 8, 4.19f, 1.92f, 0.01f},
-      {128, 64, 4, 4 + kPipelined, 8, 2.42f, 3.05f, 1.92f},
-      {64, 128, 4, 4 + kPipelined, 8, 2.89f, 3.33f, 1.6f},
-      {64, 256, 8, 3 + kPipelined, 8, 3.67f, 6.07f, 0.4f},
-      {128, 128, 4, 4 + kPipelined, 8, 3.07f, 4.73f, 2.72f},
-      {256, 128, 8, 3 + kPipelined, 8, 1.24f, 7.66f, 4.8f},
-      {128, 256, 8, 3 + kPipelined, 8, 3.0f, 8.19f, 2.94f},
-      {256, 192, 8, 2 + kPipelined, 4, 4.56f, 10.72f, 3.31f},
-      {256, 256, 8, 2 + kPipelined, 4, 2.21f, 13.15f, 4.96f}};
+// A tile's `rounds` is 0.7 times the whole rounds its workgroups make over the slots (compute units
+// times workgroups a unit) plus 0.3 times the exact ratio (a round of which a part is idle is as
+// long, but the clock is higher); where two fit a unit, one alone takes `alone` of their time.  The
+// numbers of each tile are fitted to its measured times (rms error 5-15%) on MI355X.
+//  * From 129 tokens on (33 where the plan is a macro tile already): 33 weight shapes, K
+//    1024-28672, N 1024-57344, 33-5000 tokens.  The pick takes 1.007x the fastest tile's time on
+//    the geometric mean, 1.006x over eight of the shapes left out of the fit, where the plan takes
+//    1.08-1.13x, and 1.2-1.3x at tuned shapes between their buckets (512, 1024, 2048, 4096).  So a
+//    tuned macro tile is kept up to 512 tokens, where buckets lie 8-16 tokens apart (a tuned decode
+//    tile only to 128: one token more doubles its row blocks).  The phased tiles (K a multiple
+//    of 256, from 512) beat the ring of their own size at all of these points but two, so the
+//    larger rings serve the other K.
+//  * 17-128 tokens, no tuned entry: 19 shapes, K 1024-28672, N 1536-18944, where the plan takes
+//    1.19x (20 tokens) to 1.44x (100) the fastest tile's time and the pick 1.03x.  Up to K = 2048
+//    the plan's single-step tiles are the better (or the equal), unless it fell back to streaming.
+//    The shared ring is the pick on long K, where it is up to 2.1x faster than the plan.
+// `split`: whether the caller has a workspace for a split of K.
+struct ModelTile {
+  int bm, bn, warps, stages, group_m;
+  int per_cu;                        // workgroups a compute unit holds
+  float alone, fixed, step, turn;    // us; step per 1000 bytes of K
+};
+static float modelled_us(const ModelTile& t, int64_t M, int64_t N, int64_t K, int64_t cus) {
+  const int64_t wgs = ((M + t.bm - 1) / t.bm) * (N / t.bn);
+  const int64_t slots = t.per_cu * cus, rest = wgs % slots;
+  const float last = rest == 0 ? 0.0f : t.per_cu > 1 && rest <= cus ? t.alone : 1.0f;
+  const float rounds = 0.7f * ((float)(wgs / slots) + last) + 0.3f * (float)wgs / (float)slots;
+  return t.fixed + rounds * (t.step * 1e-3f * (float)K + t.turn);
+}
+
+static void launch_config(int64_t M, int64_t N, int64_t K, bool tuned, bool split,
+                          i8l_config* c) {
+  static constexpr ModelTile kMacro[] = {
+      {256, 256, 4, kPhasedStages, 4, 1, 1.0f, 0.0f, 10.75f, 9.87f},
+      {256, 192, 4, kPhasedStages, 4, 1, 1.0f, 0.6f, 8.85f, 7.04f},
+      {256, 128, 4, kPhasedStages, 4, 1, 1.0f, 2.05f, 6.74f, 2.9f},
+      {128, 256, 4, kPhasedStages, 8, 1, 1.0f, 3.82f, 7.58f, 0.44f},
+      {128, 192, 4, kPhasedStages, 8, 1, 1.0f, 4.14f, 6.15f, 0.73f},
+      {128, 128, 4, kPhasedStages, 8, 2, 0.6f, 1.94f, 8.37f, 1.47f},
+      {64, 64, 4, 4 + kPipelined, 8, 1, 1.0f, 4.19f, 1.92f, 0.01f},
+      {128, 64, 4, 4 + kPipelined, 8, 1, 1.0f, 2.42f, 3.05f, 1.92f},
+      {64, 128, 4, 4 + kPipelined, 8, 1, 1.0f, 2.89f, 3.33f, 1.6f},
+      {64, 256, 8, 3 + kPipelined, 8, 1, 1.0f, 3.67f, 6.07f, 0.4f},
+      {128, 128, 4, 4 + kPipelined, 8, 1, 1.0f, 3.07f, 4.73f, 2.72f},
+      {256, 128, 8, 3 + kPipelined, 8, 1, 1.0f, 1.24f, 7.66f, 4.8f},
+      {128, 256, 8, 3 + kPipelined, 8, 1, 1.0f, 3.0f, 8.19f, 2.94f},
+      {256, 192, 8, 2 + kPipelined, 4, 1, 1.0f, 4.56f, 10.72f, 3.31f},
+      {256, 256, 8, 2 + kPipelined, 4, 1, 1.0f, 2.21f, 13.15f, 4.96f}};
+  static constexpr ModelTile kDecode[] = {{64, 32, 4, 3, 3, 1, 1.0f, 1.71f, 1.65f, 1.83f},
+                                          {32, 32, 4, 3, 3, 1, 1.0f, 1.46f, 1.28f, 1.34f},
+                                          {32, 64, 4, 3, 3, 1, 1.0f, 1.61f, 2.03f, 1.98f},
+                                          {32, 16, 4, 3, 3, 2, 0.5f, 2.32f, 1.72f, 0.3f},
+                                          {16, 32, 4, 3, 4, 1, 1.0f, 0.5f, 1.06f, 1.53f},
+                                          {16, 16, 4, 3, 4, 2, 0.5f, 1.78f, 1.34f, 0.29f}};
+  const int ring_bm = (int)std::min<int64_t>(128, std::max<int64_t>(32, (M + 15) / 16 * 16));
   const bool macro = dmap_index(*c) >= 0 || phased_index(*c, K) >= 0;
-  if (K % 128 != 0 || N % 64 != 0 || (M <= 128 && !macro) ||
-      (tuned && M <= (macro ? 512 : 128)))
+  if (tuned && M <= (macro ? 512 : 128)) {
+    if (ring_ok(*c, K)) c->bm = ring_bm;   // the ring's tile holds every token of the batch
     return;
+  }
+  if (K % 128 != 0 || N % 64 != 0) return;
+  const bool decode = M <= 128 && !tuned && M > 16 && (K > 2048 || c->stages == 1);
+  if (M <= 128 && !macro && !decode) return;
   const bool phased = K % 256 == 0 && K >= 512;
   const int64_t cus = cu_count();
   float best = -1.0f;
+  auto consider = [&](float us, const i8l_config& cand) {
+    if (best < 0.0f || us < best) best = us, *c = cand;
+  };
   for (const auto& t : kMacro) {
     const bool ph = t.stages == kPhasedStages;
     if (N % t.bn != 0 || (phased ? !ph && t.bm * t.bn >= 128 * 128 && t.bm > 64 : ph)) continue;
-    const int64_t tiles = ((M + t.bm - 1) / t.bm) * (N / t.bn);
-    const bool two = ph && t.bm * t.bn == 128 * 128;
-    const int64_t slots = two ? 2 * cus : cus, rest = tiles % slots;
-    const float last = rest == 0 ? 0.0f : two && rest <= cus ? 0.6f : 1.0f;
-    const float rounds = 0.7f * ((float)(tiles / slots) + last) + 0.3f * (float)tiles / (float)slots;
-    const float us = t.fixed + rounds * (t.step * 1e-3f * (float)K + t.turn);
-    if (best < 0.0f || us < best) {
-      best = us;
-      *c = i8l_config{t.bm, t.bn, 128, t.warps, t.stages, t.group_m};
-    }
+    consider(modelled_us(t, M, N, K, cus),
+             i8l_config{t.bm, t.bn, 128, t.warps, t.stages, t.group_m});
+  }
+  if (!decode) return;
+  for (const auto& t : kDecode) {
+    const i8l_config cand{t.bm, t.bn, 128, t.warps, t.stages, t.group_m};
+    if (wlds_ok(cand, K)) consider(modelled_us(t, M, N, K, cus), cand);
+  }
+  for (int z = 1; z <= (split ? 8 : 1); ++z) {   // a split of K adds the sum's launch and traffic
+    const i8l_config cand{ring_bm, 64, 128, 8, kRingStages, z};
+    if (!ring_ok(cand, K)) continue;
+    const int64_t wgs = N / 64 * z;
+    const float rounds = 0.7f * (float)((wgs + cus - 1) / cus) + 0.3f * (float)wgs / (float)cus;
+    const float steps = (float)(K / 128) / (float)z;
+    consider(2.15f + rounds * (steps * (0.2541f + 0.0023f * (float)ring_bm) + 1.82f) +
+                 (z > 1 ? 1.19f + 1.21e-6f * (float)z * (float)M * (float)N : 0.0f), cand);
   }
 }
 
@@ -246,7 +282,7 @@ extern "C" int i8l_launch_config(int64_t M, int64_t N, int64_t K, int32_t tuned,
     set_error("i8l_launch_config: cfg is NULL");
     return I8L_INVALID_ARG;
   }
-  launch_config(M, N, K, tuned != 0, cfg);
+  launch_config(M, N, K, tuned != 0, true, cfg);
   return I8L_OK;
 }
 
@@ -271,7 +307,7 @@ extern "C" int i8l_w8a8_mm_supported(int64_t M, int64_t N, int64_t K, const i8l_
     return I8L_UNSUPPORTED;
   }
   if (!stream_ok(c) && staged_index(c) < 0 && dma_index(c) < 0 && dmap_index(c) < 0 &&
-      phased_index(c, K) < 0 && !wlds_ok(c, K) && !wldsp_ok(c, K) && !wlds_split_ok(c, K)) {
+      phased_index(c, K) < 0 && !ring_ok(c, K) && !wlds_ok(c, K) && !wldsp_ok(c, K) && !wlds_split_ok(c, K)) {
     set_error("config %dx%dx%d w%d s%d g%d is not built into this library", c.bm, c.bn,
               c.bk, c.warps, c.stages, c.group_m);
     return I8L_UNSUPPORTED;
@@ -285,8 +321,7 @@ extern "C" int i8l_w8a8_mm_supported(int64_t M, int64_t N, int64_t K, const i8l_
 
 extern "C" int64_t i8l_w8a8_mm_workspace_bytes(int64_t M, int64_t N, int64_t K,
                                                const i8l_config* cfg) {
-  if (!cfg || M <= 0 || N <= 0 || !wlds_split_ok(*cfg, K)) return 0;
-  return wlds_split_workspace(*cfg, M, N);
+  return !cfg || M <= 0 || N <= 0 ? 0 : split_workspace(*cfg, M, N, K);
 }
 
 namespace i8l {
@@ -333,7 +368,9 @@ int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t*
     c = *cfg;
   } else {
     default_config(M, N, K, &c);
-    launch_config(M, N, K, false, &c);
+    // (a split into the most parts must fit the workspace, whichever is picked)
+    const bool split = ws && aligned16(ws) && ws_bytes / 32 >= M * N;
+    launch_config(M, N, K, false, split, &c);
   }
   int st = i8l_w8a8_mm_supported(M, N, K, &c);
   if (st != I8L_OK) return st;
@@ -362,9 +399,10 @@ int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t*
   // the weights-through-LDS schedules keep in-tile row offsets (< 128 token rows, < 64
   // weight rows) in 32 bits; larger strides take the generic kernel
   const bool wlds = c.stages >= 3 && c.stages <= 5 && c.bn <= 64;
+  const bool ring = ring_ok(c, K);
   const bool small_strides = stride_am <= INT32_MAX / 128 && stride_bn <= INT32_MAX / 64;
-  if (fast && wlds && small_strides && c.stages == 5) {
-    const int64_t need = wlds_split_workspace(c, M, N);
+  const int64_t need = fast && (ring || (wlds && small_strides)) ? split_workspace(c, M, N, K) : 0;
+  if (need > 0) {
     if (!ws) {
       set_error("%s: config %dx%dx%d w%d s%d g%d splits K and needs a %lld-byte workspace "
                 "(i8l_w8a8_mm_ws)", who, c.bm, c.bn, c.bk, c.warps, c.stages, c.group_m,
@@ -400,6 +438,10 @@ int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t*
     err = launch_wldsp(c, a, stride_am, b, stride_bn, e, hs);
   } else if (wlds && c.stages == 3) {
     err = launch_wlds(c, a, stride_am, b, stride_bn, e, K, hs);
+  } else if (ring && c.group_m == 1) {
+    err = launch_ring(c, a, stride_am, b, stride_bn, e, K, hs);
+  } else if (ring) {
+    err = launch_wlds_split(c, a, stride_am, b, stride_bn, e, K, (int32_t*)ws, hs);
   } else if (phased) {
     err = launch_phased(phased_index(c, K), c, a, stride_am, b, stride_bn, e, (int)K, hs);
   } else if (c.stages == 2) {

@@ -1313,8 +1313,9 @@ splitk_sum(const int32_t* __restrict__ ws, Epi e) {
   store4s<EK>(e, m, n, sum, cl, sam);
 }
 
-int64_t wlds_split_workspace(const i8l_config& c, int64_t M, int64_t N) {
-  return c.stages == 5 ? (int64_t)c.group_m * M * N * 4 : 0;
+int64_t split_workspace(const i8l_config& c, int64_t M, int64_t N, int64_t K) {
+  const bool split = wlds_split_ok(c, K) || (ring_ok(c, K) && c.group_m > 1);
+  return split ? (int64_t)c.group_m * M * N * 4 : 0;
 }
 
 bool wlds_split_ok(const i8l_config& c, int64_t K) {
@@ -1374,7 +1375,7 @@ hipError_t launch_wlds_split(const i8l_config& c, const int8_t* a, int64_t lda,
   const int mt = c.bm / 16, nc = c.bn, ks = c.bk / 64;
   hipError_t err = hipErrorInvalidValue;
 #define I8L_WLDS(MT_, NC_, KS_)                                                             \
-  if (mt == MT_ && nc == NC_ && ks == KS_) err = launch_wlds_part<MT_, NC_, KS_>(c, a, lda, b, ldb, part, K, st); else
+  if (c.stages == 5 && mt == MT_ && nc == NC_ && ks == KS_) err = launch_wlds_part<MT_, NC_, KS_>(c, a, lda, b, ldb, part, K, st); else
   I8L_WLDS(1, 16, 2) I8L_WLDS(1, 16, 4) I8L_WLDS(1, 16, 6) I8L_WLDS(1, 16, 8)
   I8L_WLDS(1, 8, 2) I8L_WLDS(1, 8, 4) I8L_WLDS(1, 8, 6) I8L_WLDS(1, 8, 8)
   I8L_WLDS(1, 4, 4) I8L_WLDS(1, 4, 8)
@@ -1386,10 +1387,15 @@ hipError_t launch_wlds_split(const i8l_config& c, const int8_t* a, int64_t lda,
   I8L_WLDS(1, 64, 2) I8L_WLDS(2, 64, 2) I8L_WLDS(4, 64, 2) I8L_WLDS(1, 64, 4) I8L_WLDS(2, 64, 4)
   {}
 #undef I8L_WLDS
+  if (c.stages == kRingStages) err = launch_ring(c, a, lda, b, ldb, part, K, st);
   if (err != hipSuccess) return err;
   switch (c.group_m) {
     case 2: return launch_splitk_sum<2>(ws, e, c.bn, st);
+    case 3: return launch_splitk_sum<3>(ws, e, c.bn, st);
     case 4: return launch_splitk_sum<4>(ws, e, c.bn, st);
+    case 5: return launch_splitk_sum<5>(ws, e, c.bn, st);
+    case 6: return launch_splitk_sum<6>(ws, e, c.bn, st);
+    case 7: return launch_splitk_sum<7>(ws, e, c.bn, st);
     case 8: return launch_splitk_sum<8>(ws, e, c.bn, st);
   }
   return hipErrorInvalidValue;

@@ -48,6 +48,8 @@ class Config:
       stages == 5: the stages-3 tile (up to 64 columns) with K split into group_m (2, 4 or 8)
         parts, one workgroup each, and the int32 partials summed by a second kernel; the
         call allocates the partials' workspace (group_m * M * N * 4 bytes).
+      stages == 6: one ring of 128-byte steps shared by 8 waves (bn 64, bk 128), as many as
+        the LDS holds; K split into group_m parts (1 to 8) as for stages 5.
     Prefill schedules (bm x bn macro tiles of 64 to 256, K in bk-byte steps, `group_m`
     rows of tiles walked together):
       stages == 2: double-buffered LDS staged through registers;
@@ -133,8 +135,8 @@ def choose_config(m: int, n: int, k: int) -> Config:
 
 def launch_config(m: int, n: int, k: int, planned: Config | None = None) -> Config:
     """The config a call without an explicit one launches (i8l_launch_config): choose_config's
-    (or `planned`, as a tuned one), and from 129 tokens on the macro tile with the least
-    modelled time where no tuned entry lies close below M."""
+    (or `planned`, as a tuned one), and from 17 tokens on the tile with the least modelled time
+    where no tuned entry lies close below M."""
     tuned = planned is not None or tuned_config(m, n, k) is not None
     p = planned or choose_config(m, n, k)
     c = _lib.CConfig(p.bm, p.bn, p.bk, p.warps, p.stages, p.group_m)

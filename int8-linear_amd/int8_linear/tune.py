@@ -63,6 +63,10 @@ DMAP_TILES = [(256, 256, 64, 8, 3), (256, 256, 64, 8, 4), (256, 256, 64, 8, 5),
               (256, 192, 128, 8, 2)]
 
 
+# The shared-ring tile (stages 6): 64 columns, 8 waves, as many token rows as the batch, K in
+# group_m parts.
+SHARED_RING = 6
+
 # (BM, BN) of the built phased tiles: 4 waves, 128-byte K steps (stages 9)
 PHASED = 9
 PHASED_TILES = [(256, 256), (256, 192), (256, 128), (128, 256), (128, 192), (128, 128)]
@@ -113,6 +117,11 @@ def candidate_configs(m: int, k: int, n: int) -> list[Config]:
             for g in (1, 2, 4):              # workgroups a compute unit
                 cfg = Config(16 * mt, nc, 64 * ks, w, 4, g)
                 if supported(m, n, k, cfg):
+                    out.append(cfg)
+        if m >= 17:
+            for parts in range(1, 9):
+                cfg = Config(max(32, -(-m // 16) * 16), 64, 128, 8, SHARED_RING, parts)
+                if n // 64 * parts <= 1024 and supported(m, n, k, cfg):
                     out.append(cfg)
         for mt, nc, ks in SPLIT_TILES:
             tiles = -(-m // (16 * mt)) * (n // nc)

@@ -461,9 +461,10 @@ def test_tuner_candidate_sets(monkeypatch):
 
 
 def test_launch_config_takes_every_planned_shape():
-    """What a call launches is built and takes the shape whatever was planned; up to 128 tokens a
-    decode plan is launched as it is, and so is a tuned macro tile up to 512; beyond, the pick does
-    not depend on the plan; shapes no macro tile divides keep their plan."""
+    """What a call launches is built and takes the shape whatever was planned; up to 16 tokens (128
+    where a wave's K is one step, or tuned) a decode plan is launched as it is, and so is a tuned
+    macro tile up to 512; beyond, the pick does not depend on the plan; shapes no macro tile
+    divides keep their plan.  A tuned shared ring gets the rows of its batch."""
     def launched(m, n, k, plan=None, tuned=0):
         p = plan or default_config(m, n, k)
         c = _lib.CConfig(p.bm, p.bn, p.bk, p.warps, p.stages, p.group_m)
@@ -475,11 +476,17 @@ def test_launch_config_takes_every_planned_shape():
             for n in (4, 48, 64, 192, 320, 2304, 5504, 57344):
                 c = launched(m, n, k)
                 assert kernel.supported(m, n, k, c), (m, n, k, c.name)
-                if m <= 128 and default_config(m, n, k).stages < 9 or k % 128 or n % 64:
-                    assert c == default_config(m, n, k), (m, n, k)
+                d = default_config(m, n, k)
+                if m <= 16 or m <= 128 and k <= 2048 and 1 < d.stages < 9 or k % 128 or n % 64:
+                    assert c == d or d.stages >= 9, (m, n, k)
+                assert c.stages != 6 or c.bm >= m
     ring, decode = Config(64, 192, 128, 4, 12, 4), Config(32, 32, 128, 16, 3, 1)
     assert launched(512, 6144, 4096, ring, 1) == ring
     assert launched(128, 4096, 2048, decode, 1) == decode
     assert launched(129, 4096, 2048, decode, 1) != decode
+    shared = Config(80, 64, 128, 8, 6, 4)
+    assert launched(75, 4096, 14336, shared, 1) == shared
+    assert launched(87, 4096, 14336, shared, 1) == Config(96, 64, 128, 8, 6, 4)
+    assert launched(100, 5120, 13824) == Config(112, 64, 128, 8, 6, 3)
     for plan in (ring, Config(256, 256, 128, 8, 10, 4), default_config(777, 6144, 4096)):
         assert launched(777, 6144, 4096, plan, 1) == Config(128, 192, 128, 4, 9, 8)
