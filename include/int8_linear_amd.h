@@ -188,10 +188,10 @@ int i8l_w8a8_mm_supported(int64_t M, int64_t N, int64_t K, const i8l_config* cfg
 int i8l_default_config(int64_t M, int64_t N, int64_t K, i8l_config* cfg_out);
 
 /* The config a call without an explicit one launches, given the one planned for it in *cfg (a
- * tuned entry with tuned != 0, else i8l_default_config's): from 17 tokens without a tuned entry
- * and from 129 with one, the tile with the least modelled time (a tuned macro tile is kept up to
- * 512 tokens).  It may split K: ask i8l_w8a8_mm_workspace_bytes.  i8l_w8a8_mm and its variants
- * apply it when their cfg is NULL, without a split.  Host-only; no counterpart in the reference. */
+ * tuned entry with tuned != 0, else i8l_default_config's): without a tuned entry, and from 129
+ * tokens with one, the tile with the least modelled time where the plan is not among the fastest (a
+ * tuned macro tile is kept up to 512 tokens).  It may split K: ask i8l_w8a8_mm_workspace_bytes.
+ * i8l_w8a8_mm and its variants apply it when their cfg is NULL, without a split.  Host-only; no counterpart in the reference. */
 int i8l_launch_config(int64_t M, int64_t N, int64_t K, int32_t tuned, i8l_config* cfg);
 
 /*

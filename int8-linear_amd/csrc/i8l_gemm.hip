@@ -193,10 +193,19 @@ void default_config(int64_t M, int64_t N, int64_t K, i8l_config* c) {
 //    tile only to 128: one token more doubles its row blocks).  The phased tiles (K a multiple
 //    of 256, from 512) beat the ring of their own size at all of these points but two, so the
 //    larger rings serve the other K.
-//  * 17-128 tokens, no tuned entry: 19 shapes, K 1024-28672, N 1536-18944, where the plan takes
-//    1.19x (20 tokens) to 1.44x (100) the fastest tile's time and the pick 1.03x.  Up to K = 2048
-//    the plan's single-step tiles are the better (or the equal), unless it fell back to streaming.
-//    The shared ring is the pick on long K, where it is up to 2.1x faster than the plan.
+//  * 33-128 tokens, no tuned entry: 19 shapes, K 1024-28672, N 1536-18944, where the plan takes
+//    1.2-1.44x the fastest tile's time and the pick 1.03x.  Up to K = 2048 the plan's single-step
+//    tiles are the better (or the equal), unless it fell back to streaming.  The shared ring is the
+//    pick on long K, where it is up to 2.1x faster than the plan.
+//  * 17-32 tokens, no tuned entry, K above 2048: the plan's 32x32 tiles are within 4% of the
+//    fastest (7168x7168 at 23 tokens: 12.1 us, the pick 13.0), so only its narrower ones, which
+//    read A once for every 8 or 16 columns, are replaced (4096x5504: 11.7 -> 7.4 us).
+//  * Up to 16 tokens, no tuned entry, K above 2048, N below 24576: a plan of 32 rows, which
+//    multiplies and stages 16 rows of nothing, gives way to a 16-row tile (5120x5120 at one token:
+//    8.9 -> 7.9 us; 13824x5120: 18.1 -> 15.2, at 16 tokens 17.7 -> 17.1); the 16-row plans stay.
+//  * A tuned split of K (the decode tile's) that takes the batch in two row blocks copies every
+//    weight byte twice, so from K = 8192 the shared ring is launched instead, which holds all
+//    tokens: 14336x4096 at 96 tokens 24.1 -> 18.9 us, at 128 23.8 -> 21.0.
 // `split`: whether the caller has a workspace for a split of K.
 struct ModelTile {
   int bm, bn, warps, stages, group_m;
@@ -235,21 +244,51 @@ static void launch_config(int64_t M, int64_t N, int64_t K, bool tuned, bool spli
                                           {32, 16, 4, 3, 3, 2, 0.5f, 2.32f, 1.72f, 0.3f},
                                           {16, 32, 4, 3, 4, 1, 1.0f, 0.5f, 1.06f, 1.53f},
                                           {16, 16, 4, 3, 4, 2, 0.5f, 1.78f, 1.34f, 0.29f}};
+  static constexpr ModelTile kSixteen[] = {{16, 32, 4, 3, 3, 2, 0.5f, 2.28f, 2.13f, 0.91f},
+                                           {16, 16, 4, 3, 4, 2, 0.5f, 2.16f, 1.17f, 0.84f},
+                                           {16, 64, 4, 3, 4, 1, 1.0f, 0.6f, 1.85f, 2.93f}};
   const int ring_bm = (int)std::min<int64_t>(128, std::max<int64_t>(32, (M + 15) / 16 * 16));
   const bool macro = dmap_index(*c) >= 0 || phased_index(*c, K) >= 0;
-  if (tuned && M <= (macro ? 512 : 128)) {
-    if (ring_ok(*c, K)) c->bm = ring_bm;   // the ring's tile holds every token of the batch
-    return;
-  }
-  if (K % 128 != 0 || N % 64 != 0) return;
-  const bool decode = M <= 128 && !tuned && M > 16 && (K > 2048 || c->stages == 1);
-  if (M <= 128 && !macro && !decode) return;
-  const bool phased = K % 256 == 0 && K >= 512;
   const int64_t cus = cu_count();
   float best = -1.0f;
   auto consider = [&](float us, const i8l_config& cand) {
     if (best < 0.0f || us < best) best = us, *c = cand;
   };
+  auto consider_rings = [&](int parts) {
+    for (int z = 1; z <= parts; ++z) {   // a split of K adds the sum's launch and traffic
+      const i8l_config cand{ring_bm, 64, 128, 8, kRingStages, z};
+      if (!ring_ok(cand, K)) continue;
+      const int64_t wgs = N / 64 * z;
+      const float rounds = 0.7f * (float)((wgs + cus - 1) / cus) + 0.3f * (float)wgs / (float)cus;
+      const float steps = (float)(K / 128) / (float)z;
+      consider(2.15f + rounds * (steps * (0.2541f + 0.0023f * (float)ring_bm) + 1.82f) +
+                   (z > 1 ? 1.19f + 1.21e-6f * (float)z * (float)M * (float)N : 0.0f), cand);
+    }
+  };
+  if (tuned && split && !macro && c->stages == 5 && c->bm < M && M <= 128 && K >= 8192 &&
+      N % 64 == 0) {
+    consider_rings(8);
+    return;
+  }
+  if (tuned && M <= (macro ? 512 : 128)) {
+    if (ring_ok(*c, K)) c->bm = ring_bm;   // the ring's tile holds every token of the batch
+    return;
+  }
+  if (K % 128 != 0 || N % 64 != 0) return;
+  const bool half = M <= 16 && c->bm > 16;      // a decode plan, half of its rows idle
+  const bool narrow = M > 16 && c->bn < 32;
+  const bool decode = !tuned && M <= 128 &&
+                      (M > 32 ? K > 2048 || c->stages == 1 : narrow && K > 2048);
+  const bool sixteen = !tuned && !macro && half && K > 2048 && N < 24576;
+  if (M <= 128 && !macro && !decode && !sixteen) return;
+  const bool phased = K % 256 == 0 && K >= 512;
+  if (sixteen) {
+    for (const auto& t : kSixteen) {
+      const i8l_config cand{t.bm, t.bn, 128, t.warps, t.stages, t.group_m};
+      if (wlds_ok(cand, K)) consider(modelled_us(t, M, N, K, cus), cand);
+    }
+    return;
+  }
   for (const auto& t : kMacro) {
     const bool ph = t.stages == kPhasedStages;
     if (N % t.bn != 0 || (phased ? !ph && t.bm * t.bn >= 128 * 128 && t.bm > 64 : ph)) continue;
@@ -261,15 +300,7 @@ static void launch_config(int64_t M, int64_t N, int64_t K, bool tuned, bool spli
     const i8l_config cand{t.bm, t.bn, 128, t.warps, t.stages, t.group_m};
     if (wlds_ok(cand, K)) consider(modelled_us(t, M, N, K, cus), cand);
   }
-  for (int z = 1; z <= (split ? 8 : 1); ++z) {   // a split of K adds the sum's launch and traffic
-    const i8l_config cand{ring_bm, 64, 128, 8, kRingStages, z};
-    if (!ring_ok(cand, K)) continue;
-    const int64_t wgs = N / 64 * z;
-    const float rounds = 0.7f * (float)((wgs + cus - 1) / cus) + 0.3f * (float)wgs / (float)cus;
-    const float steps = (float)(K / 128) / (float)z;
-    consider(2.15f + rounds * (steps * (0.2541f + 0.0023f * (float)ring_bm) + 1.82f) +
-                 (z > 1 ? 1.19f + 1.21e-6f * (float)z * (float)M * (float)N : 0.0f), cand);
-  }
+  consider_rings(split ? 8 : 1);
 }
 
 }  // namespace i8l

@@ -135,8 +135,8 @@ def choose_config(m: int, n: int, k: int) -> Config:
 
 def launch_config(m: int, n: int, k: int, planned: Config | None = None) -> Config:
     """The config a call without an explicit one launches (i8l_launch_config): choose_config's
-    (or `planned`, as a tuned one), and from 17 tokens on the tile with the least modelled time
-    where no tuned entry lies close below M."""
+    (or `planned`, as a tuned one), or the tile with the least modelled time where no tuned entry
+    lies close below M."""
     tuned = planned is not None or tuned_config(m, n, k) is not None
     p = planned or choose_config(m, n, k)
     c = _lib.CConfig(p.bm, p.bn, p.bk, p.warps, p.stages, p.group_m)

@@ -461,9 +461,9 @@ def test_tuner_candidate_sets(monkeypatch):
 
 
 def test_launch_config_takes_every_planned_shape():
-    """What a call launches is built and takes the shape whatever was planned; up to 16 tokens (128
-    where a wave's K is one step, or tuned) a decode plan is launched as it is, and so is a tuned
-    macro tile up to 512; beyond, the pick does not depend on the plan; shapes no macro tile
+    """What a call launches is built and takes the shape whatever was planned; a decode plan on
+    short K is launched as it is up to 128 tokens, and so is a tuned one, and a tuned macro tile up
+    to 512; beyond, the pick does not depend on the plan; shapes no macro tile
     divides keep their plan.  A tuned shared ring gets the rows of its batch."""
     def launched(m, n, k, plan=None, tuned=0):
         p = plan or default_config(m, n, k)
@@ -477,8 +477,9 @@ def test_launch_config_takes_every_planned_shape():
                 c = launched(m, n, k)
                 assert kernel.supported(m, n, k, c), (m, n, k, c.name)
                 d = default_config(m, n, k)
-                if m <= 16 or m <= 128 and k <= 2048 and 1 < d.stages < 9 or k % 128 or n % 64:
-                    assert c == d or d.stages >= 9, (m, n, k)
+                if m <= 128 and k <= 2048 and 1 < d.stages < 9 or k % 128 or n % 64 or \
+                        m <= 16 and d.bm == 16 or 16 < m <= 32 <= d.bn:
+                    assert c == d, (m, n, k)
                 assert c.stages != 6 or c.bm >= m
     ring, decode = Config(64, 192, 128, 4, 12, 4), Config(32, 32, 128, 16, 3, 1)
     assert launched(512, 6144, 4096, ring, 1) == ring
@@ -488,5 +489,9 @@ def test_launch_config_takes_every_planned_shape():
     assert launched(75, 4096, 14336, shared, 1) == shared
     assert launched(87, 4096, 14336, shared, 1) == Config(96, 64, 128, 8, 6, 4)
     assert launched(100, 5120, 13824) == Config(112, 64, 128, 8, 6, 3)
+    split = Config(64, 64, 128, 4, 5, 2)        # two row blocks: the ring holds them in one
+    assert launched(96, 4096, 14336, split, 1) == Config(96, 64, 128, 8, 6, 4)
+    assert launched(64, 4096, 14336, split, 1) == split
+    assert launched(96, 4096, 6144, split, 1) == split
     for plan in (ring, Config(256, 256, 128, 8, 10, 4), default_config(777, 6144, 4096)):
         assert launched(777, 6144, 4096, plan, 1) == Config(128, 192, 128, 4, 9, 8)
