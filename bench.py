@@ -122,16 +122,16 @@ def graph_time_us(fn, calls: int, windows: int = 5) -> float:
 def checked_mm(d, cfg=None, copy=None):
     """The linear of operand dict d (a_q, w_q [N,K], a_s, w_s, bias) written into an output
     buffer filled with NaN first: the same C entry point and configuration as the timed calls
-    (i8l_w8a8_mm_ws, cfg or choose_config), with the output passed in, so every element the
+    (i8l_w8a8_mm_ws, cfg or launch_config), with the output passed in, so every element the
     check reads was written by the kernel (a skipped element stays NaN and fails the check)."""
     import torch
 
     from int8_linear import _lib
-    from int8_linear.kernel import _cconfig, choose_config
+    from int8_linear.kernel import _cconfig, launch_config
     a, w = d["a_q"], d["w_q"] if copy is None else copy
     m, k = a.shape
     n = w.shape[0]
-    cfg = cfg or choose_config(m, n, k)
+    cfg = cfg or launch_config(m, n, k)
     out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=a.device)
     sa, sb = d["a_s"].reshape(-1).contiguous(), d["w_s"].reshape(-1).contiguous()
     bias = d.get("bias")
@@ -369,13 +369,13 @@ def roofline_config0(dev, launches: int = 0) -> dict:
     import torch
 
     from int8_linear import w8a8_mm
-    from int8_linear.kernel import choose_config
+    from int8_linear.kernel import launch_config
     from int8_linear.operands import operands, seed_of
     m, k, n = 16, 2048, 4096
     d = operands(m, k, n, seed_of(m, k, n), device=dev)
     copies = max(2, -(-ROTATE_BYTES // (k * n)))
     ws = [d["w_q"]] + [d["w_q"].clone() for _ in range(copies - 1)]
-    cfg = choose_config(m, n, k)
+    cfg = launch_config(m, n, k)
     reps = launches or 2 * copies
     us = graph_time_us(lambda i: w8a8_mm(d["a_q"], ws[i % copies].t(), d["a_s"], d["w_s"],
                                          torch.bfloat16), reps)
@@ -405,6 +405,10 @@ def schedule_of(cfg, k: int) -> str:
         return "gemm_wlds1p"
     if cfg.stages == 5 and cfg.bn <= 64:
         return "gemm_wlds + splitk_sum"
+    if cfg.stages == 6 and cfg.bn == 64:
+        return "gemm_ring + splitk_sum" if cfg.group_m > 1 else "gemm_ring"
+    if cfg.stages == 9:
+        return "gemm_phased"
     return "gemm_dmap" if cfg.stages >= 10 else "gemm_dma"
 
 
@@ -1024,7 +1028,7 @@ def bench_llama_decode(dev) -> dict:
     import torch
 
     from int8_linear import w8a8_mm
-    from int8_linear.kernel import choose_config
+    from int8_linear.kernel import launch_config
     from int8_linear.operands import operands, seed_of
     from int8_linear.shapes import SHAPES
     rows = []
@@ -1045,7 +1049,7 @@ def bench_llama_decode(dev) -> dict:
             us = graph_time_us(lambda i: w8a8_mm(a_q, ws[i % copies].t(), a_s, w_s,
                                                  torch.bfloat16), 2 * copies, 3)
             frac = gemm_bytes(m, k, n, False) / (us * 1e-6) / 1e9 / HBM_PEAK_GBS
-            cfg = choose_config(m, n, k)
+            cfg = launch_config(m, n, k)
             rows.append([label, m, round(us, 2), round(frac, 3), f"{schedule_of(cfg, k)} {cfg.name}"])
             log(f"llama decode {label} M={m}: {us:.2f} us, {frac:.1%} of HBM ({cfg.name})")
         del ws, d
@@ -1196,7 +1200,7 @@ def bench_prefill(dev, ms=None) -> dict:
     import torch
 
     from int8_linear import w8a8_mm
-    from int8_linear.kernel import choose_config
+    from int8_linear.kernel import launch_config
     from int8_linear.operands import quant_rows
     from int8_linear.shapes import SHAPES
     ms = ms or PREFILL_M
@@ -1230,7 +1234,7 @@ def bench_prefill(dev, ms=None) -> dict:
             rows.append([label, m, round(us, 2), round(tops, 1), round(tops / INT8_PEAK_TOPS, 3)])
             log(f"prefill {label} M={m}: {us:.1f} us {tops:.0f} TOP/s")
             if m == max(ms):
-                cfg = choose_config(m, n, k)
+                cfg = launch_config(m, n, k)
                 rec = traffic.get(label, {})
                 per_shape[label] = {
                     "bound": "mfma", "achieved": round(tops, 1), "peak": INT8_PEAK_TOPS,
@@ -1260,9 +1264,9 @@ def run_linear(dev, kn: str, m: int, config: str | None, reps: int = 3) -> dict:
     the first output is checked against float64 before the profiled launches."""
     import torch
 
-    from int8_linear.kernel import Config, choose_config, w8a8_mm
+    from int8_linear.kernel import Config, launch_config, w8a8_mm
     k, n = map(int, kn.lower().split("x"))
-    cfg = Config(*map(int, config.split(","))) if config else choose_config(m, n, k)
+    cfg = Config(*map(int, config.split(","))) if config else launch_config(m, n, k)
     g = torch.Generator().manual_seed(m * 7919 + k * 31 + n)
     copies = max(2, -(-ROTATE_BYTES // (k * n)))
     ws = [torch.randint(-127, 128, (n, k), generator=g, dtype=torch.int8).to(dev)
