@@ -1,4 +1,4 @@
-// Shared-ring schedule of the W8A8 GEMM for batches of 33 to 128 tokens on long K
+// Shared-ring schedule of the W8A8 GEMM for batches of 17 to 128 tokens on long K
 // (v_mfma_i32_16x16x64_i8).
 #include "i8l_gemm_tile.h"
 

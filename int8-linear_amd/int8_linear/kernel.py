@@ -298,7 +298,7 @@ def w8a8_mm_noalloc(a_q: torch.Tensor, b_q: torch.Tensor, scale_a: torch.Tensor,
     allocate (code under HIP graph capture, serving loops that forbid it).  It has no
     counterpart in the reference.
 
-    A split of K (stages 5) keeps its int32 partial planes in the library's own 16 MiB device
+    A split of K (stages 5, 6) keeps its int32 partial planes in the library's own 16 MiB device
     array of the GPU, which every call of this entry on that GPU shares.  Calls that can
     overlap in time on one GPU (launched on two streams with no ordering between them) race
     on it and give wrong results: order them (one stream, or events).  Configurations whose
