@@ -51,14 +51,19 @@ enum {
  *                K step a wave, each workgroup walking several column tiles with the
  *                activations held in registers (decode, K == bk * warps); 5 the stages-3
  *                tile with K split over group_m workgroups and their int32 partials summed
- *                by a second kernel (decode; needs a workspace, see i8l_w8a8_mm_ws); 2 LDS
- *                staged through registers, 3..8 a ring of that many direct-to-LDS buffers,
- *                >= 10 a ring of stages - 8 buffers (2: a double buffer) with fragment reads
+ *                by a second kernel (decode; needs a workspace, see i8l_w8a8_mm_ws); 6 with
+ *                bn 64 one ring of 128-byte steps shared by 8 waves, bm (32 to 128, a multiple
+ *                of 16) token rows a workgroup (decode on long K; splits K as stages 5 does);
+ *                2 LDS staged through registers, 3..8 with bm >= 128 and bn >= 128 a ring of
+ *                that many direct-to-LDS buffers, 9 persistent macro tiles of 4 waves whose
+ *                steps are cut into four phases (K a multiple of 2 * bk, from 4 * bk on), >= 10
+ *                a ring of stages - 8 buffers (2: a double buffer) with fragment reads
  *                overlapped with the MFMAs (prefill)
  *   group_m    : rows of tiles walked together for L2 reuse (1 = row-major order); stages 3
  *                with bn <= 64: 3 keeps two K steps in flight (three step buffers a
- *                wave), 4 three (four buffers), else one; with stages 4, the workgroups a compute unit runs at once (1, 2 or 4); with
- *                stages 5, the parts K is split into (2, 4 or 8)
+ *                wave), 4 three (four buffers), else one; with stages 4, the workgroups a
+ *                compute unit runs at once (1, 2 or 4); with stages 5, the parts K is split
+ *                into (2, 4 or 8), with stages 6 and bn 64 too (1 to 8, 1 no split)
  * A config the library was not built for returns I8L_UNSUPPORTED.
  */
 typedef struct i8l_config {
@@ -77,10 +82,11 @@ typedef struct i8l_config {
  * correct generic kernel.  scale_a has scale_a_len 1 or M fp32 values, scale_b has 1 or N.
  * bias is NULL (bias_dtype I8L_DTYPE_NONE) or N values of bf16/f16/f32.  out is [M,N] with
  * row stride stride_cm and unit column stride, of out_dtype bf16/f16/f32/i32.
- * cfg NULL picks the library default for (M,N,K).
+ * cfg NULL is i8l_default_config's for (M,N,K) as i8l_launch_config then changes it, but never
+ * a split of K.
  *
- * A config that splits K (stages 5) needs a workspace: this entry declines it with
- * I8L_UNSUPPORTED; i8l_w8a8_mm_ws takes it.
+ * A config that splits K (stages 5, or 6 with group_m > 1) needs a workspace: this entry
+ * declines it with I8L_UNSUPPORTED; i8l_w8a8_mm_ws takes it.
  *
  * Replaces the reference's launch of the Triton kernel _w8a8_mm from
  * w8a8_mm (int8_linear/kernel.py:202-257; kernel body 63-124).
@@ -96,8 +102,9 @@ int i8l_w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak,
 
 /*
  * Bytes of device workspace that i8l_w8a8_mm_ws needs for (M,N,K,cfg): group_m * M * N * 4
- * for a split of K (stages 5: one int32 partial plane per part), 0 for every other
- * schedule and for cfg NULL (the default config never splits).  Host-only; always >= 0.
+ * for a split of K (stages 5, or 6 with group_m > 1: one int32 partial plane per part), 0 for
+ * every other schedule and for cfg NULL (a call without a config never splits).  Host-only;
+ * always >= 0.
  * Replaces nothing in the reference (its Triton kernel keeps the whole K loop in one
  * program, int8_linear/kernel.py:94-103); it sizes the buffer the caller allocates.
  */
@@ -110,7 +117,7 @@ int64_t i8l_w8a8_mm_workspace_bytes(int64_t M, int64_t N, int64_t K, const i8l_c
  * matter, and on return they are undefined.  Calls in flight at the same time must not
  * share a workspace.  A workspace smaller than needed returns I8L_INVALID_ARG.
  * Replaces the same reference launch as i8l_w8a8_mm (int8_linear/kernel.py:202-257), with
- * the kernel's K loop (kernel.py:94-103) split across workgroups for stages 5.
+ * the kernel's K loop (kernel.py:94-103) split across workgroups for stages 5 and 6.
  */
 int i8l_w8a8_mm_ws(const int8_t* a, int64_t stride_am, int64_t stride_ak,
                    const int8_t* b, int64_t stride_bk, int64_t stride_bn,
@@ -150,7 +157,7 @@ int i8l_w8a8_mm_silu_mul_supported(int64_t M, int64_t N, int64_t K, const i8l_co
  * i8l_w8a8_mm for callers that cannot allocate: code under HIP graph capture, serving loops
  * and harnesses that forbid allocation.  No counterpart in the reference (its Triton kernel
  * needs no workspace).  Same arguments, validation and results as i8l_w8a8_mm_ws, but a
- * split of K (stages 5) keeps its partial planes in a device array of the library itself,
+ * split of K (stages 5, 6) keeps its partial planes in a device array of the library itself,
  * 16 MiB on each GPU it runs on (held until the process ends); a config that needs more
  * (group_m * M * N * 4 bytes > 16 MiB) returns I8L_UNSUPPORTED.  No call allocates or frees
  * memory.  All calls on one GPU share that array: calls that overlap in time on one GPU race.
@@ -191,7 +198,8 @@ int i8l_default_config(int64_t M, int64_t N, int64_t K, i8l_config* cfg_out);
  * tuned entry with tuned != 0, else i8l_default_config's): without a tuned entry, and from 129
  * tokens with one, the tile with the least modelled time where the plan is not among the fastest (a
  * tuned macro tile is kept up to 512 tokens).  It may split K: ask i8l_w8a8_mm_workspace_bytes.
- * i8l_w8a8_mm and its variants apply it when their cfg is NULL, without a split.  Host-only; no counterpart in the reference. */
+ * i8l_w8a8_mm, i8l_w8a8_mm_ws and i8l_w8a8_mm_noalloc apply it when their cfg is NULL, but never
+ * pick a split there.  Host-only; no counterpart in the reference. */
 int i8l_launch_config(int64_t M, int64_t N, int64_t K, int32_t tuned, i8l_config* cfg);
 
 /*

@@ -206,7 +206,7 @@ void default_config(int64_t M, int64_t N, int64_t K, i8l_config* c) {
 //  * A tuned split of K (the decode tile's) that takes the batch in two row blocks copies every
 //    weight byte twice, so from K = 8192 the shared ring is launched instead, which holds all
 //    tokens: 14336x4096 at 96 tokens 24.1 -> 18.9 us, at 128 23.8 -> 21.0.
-// `split`: whether the caller has a workspace for a split of K.
+// `split`: whether a split of K may be picked (a caller that asks for its workspace afterwards).
 struct ModelTile {
   int bm, bn, warps, stages, group_m;
   int per_cu;                        // workgroups a compute unit holds
@@ -398,10 +398,10 @@ int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t*
   if (cfg) {
     c = *cfg;
   } else {
+    // never a split of K: i8l_w8a8_mm_workspace_bytes gives 0 for no config, so a workspace that
+    // is passed all the same may be shared by calls in flight
     default_config(M, N, K, &c);
-    // (a split into the most parts must fit the workspace, whichever is picked)
-    const bool split = ws && aligned16(ws) && ws_bytes / 32 >= M * N;
-    launch_config(M, N, K, false, split, &c);
+    launch_config(M, N, K, false, false, &c);
   }
   int st = i8l_w8a8_mm_supported(M, N, K, &c);
   if (st != I8L_OK) return st;

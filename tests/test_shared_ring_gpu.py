@@ -90,3 +90,25 @@ def test_no_split_without_a_workspace():
     assert torch.equal(out, w8a8_mm(a, w.t(), sa, sb))
     c = kernel._cconfig(Config(112, 64, 128, 8, 6, 3))
     assert _lib.lib().i8l_w8a8_mm_workspace_bytes(m, n, k, c) == 3 * m * n * 4
+
+
+@pytest.mark.parametrize("m,k,n", [(48, 13824, 5120), (75, 18944, 3584), (100, 13824, 5120)])
+def test_no_config_leaves_a_workspace_alone(m, k, n):
+    """i8l_w8a8_mm_ws without a configuration does not split K, however large the workspace it is
+    handed: i8l_w8a8_mm_workspace_bytes gives 0 for such a call, so several in flight may share
+    one."""
+    say(f"ws with no config m={m} k={k} n={n}")
+    a, w = ints((m, k), 7), ints((n, k), 8)
+    sa, sb = torch.rand(m).cuda() * 1e-2, torch.rand(n).cuda() * 1e-2
+    assert kernel.launch_config(m, n, k).group_m > 1      # the pick with a workspace
+    lib = _lib.lib()
+    assert lib.i8l_w8a8_mm_workspace_bytes(m, n, k, None) == 0
+    ws = torch.full((32 * m * n,), 0x5a, dtype=torch.uint8, device="cuda")
+    out = torch.empty((m, n), dtype=torch.bfloat16, device="cuda")
+    status = lib.i8l_w8a8_mm_ws(a.data_ptr(), k, 1, w.data_ptr(), 1, k, sa.data_ptr(), m,
+                                sb.data_ptr(), n, None, _lib.DTYPE_NONE, out.data_ptr(), n,
+                                _lib.BF16, m, n, k, ws.data_ptr(), ws.numel(), None,
+                                _lib.stream_of(a))
+    assert status == _lib.OK, _lib.last_error()
+    assert torch.equal(out, w8a8_mm(a, w.t(), sa, sb))
+    assert bool((ws == 0x5a).all())
