@@ -447,9 +447,11 @@ int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t*
     }
   }
   hipError_t err;
-  // the phased schedule keeps in-tile offsets (256 rows of either operand) in 32 bits
+  // the phased schedule keeps in-tile offsets (256 rows of either operand) in unsigned 32 bits,
+  // so it takes no rows in reverse either
   const bool phased = c.stages == kPhasedStages;
-  const bool phased_strides = stride_am <= INT32_MAX / 256 && stride_bn <= INT32_MAX / 256;
+  const bool phased_strides = stride_am >= 0 && stride_am <= INT32_MAX / 256 &&
+                              stride_bn >= 0 && stride_bn <= INT32_MAX / 256;
   if (!fast || (wlds && !small_strides) || (phased && !phased_strides)) {
     const int64_t tiles = ((N + 63) / 64) * ((M + 63) / 64);
     if (tiles > INT32_MAX) {

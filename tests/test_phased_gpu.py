@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from helpers import bits, ints, np_, say
-from int8_linear import Config, kernel, tune, w8a8_mm
+from int8_linear import Config, _lib, kernel, tune, w8a8_mm
 from oracle import oracle as o
 
 pytestmark = pytest.mark.gpu
@@ -79,6 +79,28 @@ def test_wide_strides_take_the_generic_kernel():
     one = torch.ones(1, device="cuda")
     got = w8a8_mm(view, w.t(), one, one, raw=True, config=config)
     assert np.array_equal(np_(got), o.gemm_i32(np_(a), np_(w)))
+
+
+@pytest.mark.parametrize("config", [None, *TILES], ids=lambda c: c.name if c else "none")
+@pytest.mark.parametrize("which", ["a", "b", "both"])
+def test_rows_in_reverse(config, which):
+    """Row strides below 0 through the C entry (a base at the last row): the phased kernel's in-tile
+    offsets are unsigned, so such a call leaves it."""
+    m, k, n = 300, 512, 2 * (config.bn if config else 192)
+    say(f"reversed rows {which} {config.name if config else None}")
+    a, w = ints((m, k), 9), ints((n, k), 10)
+    one = torch.ones(1, device="cuda")
+    out = torch.empty((m, n), dtype=torch.int32, device="cuda")
+    ra, rb = which != "b", which != "a"
+    lib = _lib.lib()
+    status = lib.i8l_w8a8_mm(
+        a.data_ptr() + (m - 1) * k * ra, -k if ra else k, 1,
+        w.data_ptr() + (n - 1) * k * rb, 1, -k if rb else k, one.data_ptr(), 1, one.data_ptr(), 1,
+        None, _lib.DTYPE_NONE, out.data_ptr(), n, _lib.I32, m, n, k,
+        kernel._cconfig(config) if config else None, _lib.stream_of(a))
+    assert status == _lib.OK, _lib.last_error()
+    ref = o.gemm_i32(np_(a)[::-1] if ra else np_(a), np_(w)[::-1] if rb else np_(w))
+    assert np.array_equal(np_(out), ref)
 
 
 @pytest.mark.parametrize("m,k,n", [(129, 512, 640), (300, 2752, 5504), (777, 4096, 1536),
