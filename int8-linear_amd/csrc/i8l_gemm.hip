@@ -357,6 +357,17 @@ extern "C" int64_t i8l_w8a8_mm_workspace_bytes(int64_t M, int64_t N, int64_t K,
 
 namespace i8l {
 
+// Whether a config's schedule takes these row strides.  The weights-through-LDS schedules keep
+// in-tile row offsets (< 128 token rows, < 64 weight rows) in 32 bits, the phased one (< 256 rows
+// of either operand) in unsigned 32 bits, so no stride below 0; the others address in 64.
+static bool strides_ok(const i8l_config& c, int64_t lda, int64_t ldb) {
+  if (c.stages == kPhasedStages)
+    return lda >= 0 && ldb >= 0 && lda <= INT32_MAX / 256 && ldb <= INT32_MAX / 256;
+  if (c.stages >= 3 && c.stages <= 5 && c.bn <= 64)
+    return std::abs(lda) <= INT32_MAX / 128 && std::abs(ldb) <= INT32_MAX / 64;
+  return true;
+}
+
 // The GEMM behind every entry point: validation, then the schedule of the config.  `ws` is
 // the split of K's workspace (NULL, 0 when the caller has none).
 int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t* b,
@@ -427,12 +438,21 @@ int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t*
                     (stride_cm * osz) % 16 == 0 && stride_cm >= N && N % 4 == 0 &&
                     (e.sb_per_col == 0 || aligned16(scale_b)) &&
                     (e.bias_dtype == I8L_DTYPE_NONE || aligned16(bias));
-  // the weights-through-LDS schedules keep in-tile row offsets (< 128 token rows, < 64
-  // weight rows) in 32 bits; larger strides take the generic kernel
+  // Strides that the schedule does not take go to the default plan's, which from 129 tokens on
+  // takes any, or else to the generic kernel (200 x 9728 x 2560 with 8 MiB between token rows: 33
+  // us against 238).
+  bool strides = strides_ok(c, stride_am, stride_bn);
+  if (fast && !strides) {
+    i8l_config plan;
+    default_config(M, N, K, &plan);
+    strides = strides_ok(plan, stride_am, stride_bn) &&
+              i8l_w8a8_mm_supported(M, N, K, &plan) == I8L_OK;
+    if (strides) c = plan;
+  }
   const bool wlds = c.stages >= 3 && c.stages <= 5 && c.bn <= 64;
   const bool ring = ring_ok(c, K);
-  const bool small_strides = stride_am <= INT32_MAX / 128 && stride_bn <= INT32_MAX / 64;
-  const int64_t need = fast && (ring || (wlds && small_strides)) ? split_workspace(c, M, N, K) : 0;
+  const int64_t need =
+      fast && strides && (ring || wlds) ? split_workspace(c, M, N, K) : 0;
   if (need > 0) {
     if (!ws) {
       set_error("%s: config %dx%dx%d w%d s%d g%d splits K and needs a %lld-byte workspace "
@@ -447,12 +467,7 @@ int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t*
     }
   }
   hipError_t err;
-  // the phased schedule keeps in-tile offsets (256 rows of either operand) in unsigned 32 bits,
-  // so it takes no rows in reverse either
-  const bool phased = c.stages == kPhasedStages;
-  const bool phased_strides = stride_am >= 0 && stride_am <= INT32_MAX / 256 &&
-                              stride_bn >= 0 && stride_bn <= INT32_MAX / 256;
-  if (!fast || (wlds && !small_strides) || (phased && !phased_strides)) {
+  if (!fast || !strides) {
     const int64_t tiles = ((N + 63) / 64) * ((M + 63) / 64);
     if (tiles > INT32_MAX) {
       set_error("%s: %lld x %lld is too large for the generic kernel", who, (long long)M,
@@ -475,7 +490,7 @@ int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t*
     err = launch_ring(c, a, stride_am, b, stride_bn, e, K, hs);
   } else if (ring) {
     err = launch_wlds_split(c, a, stride_am, b, stride_bn, e, K, (int32_t*)ws, hs);
-  } else if (phased) {
+  } else if (c.stages == kPhasedStages) {
     err = launch_phased(phased_index(c, K), c, a, stride_am, b, stride_bn, e, (int)K, hs);
   } else if (c.stages == 2) {
     err = launch_staged(staged_index(c), c, a, stride_am, b, stride_bn, e, (int)K, hs);

@@ -67,7 +67,7 @@ def test_every_bias_and_scale(config, dtype):
             assert np.array_equal(out, ref), (per_row, per_col, bd)
 
 
-def test_wide_strides_take_the_generic_kernel():
+def test_wide_strides_leave_the_phased_kernel():
     """Row strides past what 32-bit in-tile offsets hold (256 rows) leave the phased kernel."""
     config, m, k, n = TILES[0], 3, 512, 256
     stride = (2 ** 31 - 1) // 256 + 1 + 15 & ~15
@@ -79,6 +79,38 @@ def test_wide_strides_take_the_generic_kernel():
     one = torch.ones(1, device="cuda")
     got = w8a8_mm(view, w.t(), one, one, raw=True, config=config)
     assert np.array_equal(np_(got), o.gemm_i32(np_(a), np_(w)))
+
+
+def test_wide_strides_keep_the_plan():
+    """A call without a configuration whose token rows lie further apart than the phased tile it
+    would launch takes runs the default plan, not the generic kernel, which is nine times slower here
+    than packed rows (the plan 1.3 times): three times is allowed."""
+    m, k, n = 200, 2560, 9728
+    stride = (2 ** 31 - 1) // 256 + 1 + 15 & ~15
+    assert kernel.launch_config(m, n, k).stages == tune.PHASED
+    say(f"no config, wide stride {stride}")
+    a, w = ints((m, k), 7), ints((n, k), 8)
+    wide = torch.zeros((m - 1) * stride + k, dtype=torch.int8, device="cuda")
+    view = wide.as_strided((m, k), (stride, 1))
+    view.copy_(a)
+    one = torch.ones(1, device="cuda")
+    ref = o.gemm_i32(np_(a), np_(w))
+
+    def us(x):
+        best = float("inf")
+        for _ in range(10):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            got = w8a8_mm(x, w.t(), one, one, raw=True)
+            e1.record()
+            e1.synchronize()
+            best = min(best, e0.elapsed_time(e1) * 1e3)
+        assert np.array_equal(np_(got), ref)
+        return best
+
+    packed, apart = us(a), us(view)
+    say(f"{packed:.1f} us packed, {apart:.1f} us apart")
+    assert apart < 3 * packed, (packed, apart)
 
 
 @pytest.mark.parametrize("config", [None, *TILES], ids=lambda c: c.name if c else "none")
