@@ -194,13 +194,17 @@ int i8l_w8a8_mm_supported(int64_t M, int64_t N, int64_t K, const i8l_config* cfg
  * int8_linear/kernel.py:127-134, re-derived for MI355X). Host-only. */
 int i8l_default_config(int64_t M, int64_t N, int64_t K, i8l_config* cfg_out);
 
-/* The config a call without an explicit one launches, given the one planned for it in *cfg (a
- * tuned entry with tuned != 0, else i8l_default_config's): without a tuned entry, and from 129
- * tokens with one, the tile with the least modelled time where the plan is not among the fastest (a
- * tuned macro tile is kept up to 512 tokens).  It may split K: ask i8l_w8a8_mm_workspace_bytes.
- * i8l_w8a8_mm, i8l_w8a8_mm_ws and i8l_w8a8_mm_noalloc apply it when their cfg is NULL, but never
- * pick a split there.  Host-only; no counterpart in the reference. */
-int i8l_launch_config(int64_t M, int64_t N, int64_t K, int32_t tuned, i8l_config* cfg);
+/* The config a call without an explicit one launches, given the one planned for it in *cfg: a tuned
+ * entry, with tuned_m the token count it was tuned at, or i8l_default_config's with tuned_m 0.  A
+ * tuned entry is kept up to 128 tokens (a macro tile up to 512), and beyond while the M tokens make
+ * as many row blocks of bm as its own tuned_m, so always at M == tuned_m.  (Two changes below that:
+ * a shared ring, stages 6, gets the rows of the batch; from K = 8192 an entry that splits K and needs
+ * more row blocks than at tuned_m gives way to one.)  Without a tuned entry, and past those
+ * bounds, it is the tile with the least modelled time where the plan is not among the fastest.  It
+ * may split K: ask i8l_w8a8_mm_workspace_bytes.  i8l_w8a8_mm, i8l_w8a8_mm_ws and
+ * i8l_w8a8_mm_noalloc apply it when their cfg is NULL, with no tuned entry, and never pick a split
+ * there.  Host-only; no counterpart in the reference. */
+int i8l_launch_config(int64_t M, int64_t N, int64_t K, int32_t tuned_m, i8l_config* cfg);
 
 /*
  * Fused add + RMSNorm + per-token int8 quantize, one row per token:

@@ -189,8 +189,10 @@ void default_config(int64_t M, int64_t N, int64_t K, i8l_config* c) {
 //    1024-28672, N 1024-57344, 33-5000 tokens.  The pick takes 1.007x the fastest tile's time on
 //    the geometric mean, 1.006x over eight of the shapes left out of the fit, where the plan takes
 //    1.08-1.13x, and 1.2-1.3x at tuned shapes between their buckets (512, 1024, 2048, 4096).  So a
-//    tuned macro tile is kept up to 512 tokens, where buckets lie 8-16 tokens apart (a tuned decode
-//    tile only to 128: one token more doubles its row blocks).  The phased tiles (K a multiple
+//    tuned macro tile is kept up to 512 tokens, where buckets lie 8-16 tokens apart, and a tuned
+//    decode tile up to 128.  Beyond, an entry is kept while the batch makes the row blocks that it
+//    was measured with, so at its own token count always: 2048x1024 at 144 tokens 5.5 us in 9
+//    blocks of 16 rows, 8.1 at 145 in 10, the pick 7.2.  The phased tiles (K a multiple
 //    of 256, from 512) beat the ring of their own size at all of these points but two, so the
 //    larger rings serve the other K.
 //  * 33-128 tokens, no tuned entry: 19 shapes, K 1024-28672, N 1536-18944, where the plan takes
@@ -203,9 +205,11 @@ void default_config(int64_t M, int64_t N, int64_t K, i8l_config* c) {
 //  * Up to 16 tokens, no tuned entry, K above 2048, N below 24576: a plan of 32 rows, which
 //    multiplies and stages 16 rows of nothing, gives way to a 16-row tile (5120x5120 at one token:
 //    8.9 -> 7.9 us; 13824x5120: 18.1 -> 15.2, at 16 tokens 17.7 -> 17.1); the 16-row plans stay.
-//  * A tuned split of K (the decode tile's) that takes the batch in two row blocks copies every
-//    weight byte twice, so from K = 8192 the shared ring is launched instead, which holds all
-//    tokens: 14336x4096 at 96 tokens 24.1 -> 18.9 us, at 128 23.8 -> 21.0.
+//  * A tuned split of K (the decode tile's) for fewer tokens that takes the batch in more row
+//    blocks than it was tuned with copies every weight byte once for each, so from K = 8192 the
+//    shared ring is launched instead, which holds all tokens: 14336x4096 at 96 tokens 24.1 ->
+//    18.9 us, at 128 23.8 -> 21.0.
+// `tuned`: the token count that the planned entry was tuned at, 0 for none.
 // `split`: whether a split of K may be picked (a caller that asks for its workspace afterwards).
 struct ModelTile {
   int bm, bn, warps, stages, group_m;
@@ -220,7 +224,7 @@ static float modelled_us(const ModelTile& t, int64_t M, int64_t N, int64_t K, in
   return t.fixed + rounds * (t.step * 1e-3f * (float)K + t.turn);
 }
 
-static void launch_config(int64_t M, int64_t N, int64_t K, bool tuned, bool split,
+static void launch_config(int64_t M, int64_t N, int64_t K, int64_t tuned, bool split,
                           i8l_config* c) {
   static constexpr ModelTile kMacro[] = {
       {256, 256, 4, kPhasedStages, 4, 1, 1.0f, 0.0f, 10.75f, 9.87f},
@@ -265,12 +269,14 @@ static void launch_config(int64_t M, int64_t N, int64_t K, bool tuned, bool spli
                    (z > 1 ? 1.19f + 1.21e-6f * (float)z * (float)M * (float)N : 0.0f), cand);
     }
   };
-  if (tuned && split && !macro && c->stages == 5 && c->bm < M && M <= 128 && K >= 8192 &&
-      N % 64 == 0) {
+  auto blocks = [&](int64_t m) { return (m + c->bm - 1) / c->bm; };
+  const bool as_tuned = tuned > 0 && c->bm > 0 && blocks(M) == blocks(tuned);
+  if (tuned && !as_tuned && split && c->stages == 5 && c->bm < M && M <= 128 && K >= 8192 &&
+      N % 64 == 0 && !macro) {
     consider_rings(8);
     return;
   }
-  if (tuned && M <= (macro ? 512 : 128)) {
+  if (tuned && (M <= (macro ? 512 : 128) || (as_tuned && tuned > 128))) {
     if (ring_ok(*c, K)) c->bm = ring_bm;   // the ring's tile holds every token of the batch
     return;
   }
@@ -307,13 +313,13 @@ static void launch_config(int64_t M, int64_t N, int64_t K, bool tuned, bool spli
 
 using namespace i8l;
 
-extern "C" int i8l_launch_config(int64_t M, int64_t N, int64_t K, int32_t tuned,
+extern "C" int i8l_launch_config(int64_t M, int64_t N, int64_t K, int32_t tuned_m,
                                  i8l_config* cfg) {
   if (!cfg) {
     set_error("i8l_launch_config: cfg is NULL");
     return I8L_INVALID_ARG;
   }
-  launch_config(M, N, K, tuned != 0, true, cfg);
+  launch_config(M, N, K, tuned_m, true, cfg);
   return I8L_OK;
 }
 
@@ -412,7 +418,7 @@ int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t*
     // never a split of K: i8l_w8a8_mm_workspace_bytes gives 0 for no config, so a workspace that
     // is passed all the same may be shared by calls in flight
     default_config(M, N, K, &c);
-    launch_config(M, N, K, false, false, &c);
+    launch_config(M, N, K, 0, false, &c);
   }
   int st = i8l_w8a8_mm_supported(M, N, K, &c);
   if (st != I8L_OK) return st;

@@ -73,16 +73,19 @@ void set_table(int device, const std::vector<std::vector<int64_t>>& rows) {
 
 bool has_table(int device) { return g_tables.count(device) != 0; }
 
-// false when the device's table has not been handed over yet; *tuned: c is a table entry
-bool choose(int device, int64_t m, int64_t n, int64_t k, i8l_config* c, bool* tuned = nullptr) {
+// false when the device's table has not been handed over yet; *tuned_m: the entry's bucket, 0 when
+// c is not a table entry
+bool choose(int device, int64_t m, int64_t n, int64_t k, i8l_config* c, int32_t* tuned_m) {
+  *tuned_m = 0;
   auto dt = g_tables.find(device);
   if (dt == g_tables.end()) return false;
   auto st = dt->second.shapes.find(kn_key(k, n));
   if (st != dt->second.shapes.end()) {
     auto it = st->second.upper_bound(m);  // first bucket above M
     if (it != st->second.begin()) {
-      *c = std::prev(it)->second;
-      if (tuned) *tuned = true;
+      --it;
+      *c = it->second;
+      *tuned_m = (int32_t)it->first;
       return true;
     }
   }
@@ -93,7 +96,18 @@ bool choose(int device, int64_t m, int64_t n, int64_t k, i8l_config* c, bool* tu
 // or None before the device's table is handed over.
 py::object config_for(int device, int64_t m, int64_t n, int64_t k) {
   i8l_config c;
-  if (!choose(device, m, n, k, &c)) return py::none();
+  int32_t tuned_m;
+  if (!choose(device, m, n, k, &c, &tuned_m)) return py::none();
+  return py::make_tuple(c.bm, c.bn, c.bk, c.warps, c.stages, c.group_m);
+}
+
+// The configuration mm launches, likewise.
+py::object launch_config_for(int device, int64_t m, int64_t n, int64_t k) {
+  i8l_config c;
+  int32_t tuned_m;
+  if (!choose(device, m, n, k, &c, &tuned_m) ||
+      i8l_launch_config(m, n, k, tuned_m, &c) != I8L_OK)
+    return py::none();
   return py::make_tuple(c.bm, c.bn, c.bk, c.warps, c.stages, c.group_m);
 }
 
@@ -134,9 +148,10 @@ py::object mm(const at::Tensor& a, const at::Tensor& b, const at::Tensor& sa,
   const int64_t m = a.size(0), k = a.size(1), n = b.size(1);
   if (b.size(0) != k || b.device() != dev) return py::none();
   i8l_config c;
-  bool tuned = false;
-  if (!choose(dev.index(), m, n, k, &c, &tuned) ||
-      i8l_launch_config(m, n, k, tuned ? 1 : 0, &c) != I8L_OK || c.bn <= 0 || c.bk <= 0 || n % c.bn || k % c.bk)
+  int32_t tuned_m;
+  if (!choose(dev.index(), m, n, k, &c, &tuned_m) ||
+      i8l_launch_config(m, n, k, tuned_m, &c) != I8L_OK || c.bn <= 0 || c.bk <= 0 ||
+      n % c.bn || k % c.bk)
     return py::none();
   if (!plain_vector(sa, at::kFloat, dev) || !plain_vector(sb, at::kFloat, dev)) return py::none();
   if ((sa.numel() != 1 && sa.numel() != m) || (sb.numel() != 1 && sb.numel() != n))
@@ -243,6 +258,7 @@ PYBIND11_MODULE(_i8l_fast, m) {
   m.def("set_table", &set_table, "hand over one device's tuned configurations");
   m.def("has_table", &has_table);
   m.def("config_for", &config_for);
+  m.def("launch_config_for", &launch_config_for);
   m.def("launches", [] { return g_launches; });
   m.def("mm", &mm, py::arg("a_q"), py::arg("b_q"), py::arg("scale_a"), py::arg("scale_b"),
         py::arg("out_dtype"), py::arg("bias"));

@@ -113,12 +113,20 @@ def _device_table(device: int) -> dict:
     return table
 
 
+def tuned_bucket(m: int, n: int, k: int) -> int:
+    """The largest tuned batch bucket of this GPU and shape at or below M, 0 if there is none."""
+    table = _device_table(torch.cuda.current_device()).get(f"{k}x{n}", {})
+    return max((int(bucket) for bucket in table if int(bucket) <= m), default=0)
+
+
 def tuned_config(m: int, n: int, k: int) -> Config | None:
     """The fastest measured config for this GPU and shape, from the largest tuned batch
     bucket at or below M, or None if nothing has been tuned (reference kernel.py:143-148)."""
-    table = _device_table(torch.cuda.current_device()).get(f"{k}x{n}", {})
-    fits = [int(bucket) for bucket in table if int(bucket) <= m]
-    return Config(**table[str(max(fits))]["config"]) if fits else None
+    bucket = tuned_bucket(m, n, k)
+    if not bucket:
+        return None
+    table = _device_table(torch.cuda.current_device())
+    return Config(**table[f"{k}x{n}"][str(bucket)]["config"])
 
 
 _chosen: dict[tuple[int, int, int, int], Config] = {}
@@ -135,12 +143,12 @@ def choose_config(m: int, n: int, k: int) -> Config:
 
 def launch_config(m: int, n: int, k: int, planned: Config | None = None) -> Config:
     """The config a call without an explicit one launches (i8l_launch_config): choose_config's
-    (or `planned`, as a tuned one), or the tile with the least modelled time where no tuned entry
-    lies close below M."""
-    tuned = planned is not None or tuned_config(m, n, k) is not None
+    (or `planned`, as one tuned for a single token), or the tile with the least modelled time where
+    no tuned entry lies close below M.  A tuned entry is always launched at its own token count."""
+    bucket = 1 if planned is not None else tuned_bucket(m, n, k)
     p = planned or choose_config(m, n, k)
     c = _lib.CConfig(p.bm, p.bn, p.bk, p.warps, p.stages, p.group_m)
-    _lib.check(_lib.lib().i8l_launch_config(m, n, k, int(tuned), c), NotSupported)
+    _lib.check(_lib.lib().i8l_launch_config(m, n, k, bucket, c), NotSupported)
     return Config(c.bm, c.bn, c.bk, c.warps, c.stages, c.group_m)
 
 

@@ -4,6 +4,7 @@ and its host-only entry points (config choice, the decline rule) behave.  CPU on
 from __future__ import annotations
 
 import ctypes
+import json
 import re
 from pathlib import Path
 
@@ -458,6 +459,48 @@ def test_tuner_candidate_sets(monkeypatch):
     assert not any(map(split, tune.candidate_configs(128, 4096, 28672)))
     assert tune.parse_ms("capture") == list(tune.CAPTURE_SIZES)
     assert tune.parse_ms("1,2,17") == [1, 2, 17]
+
+
+def _launched(m, n, k, plan, tuned):
+    c = _lib.CConfig(plan.bm, plan.bn, plan.bk, plan.warps, plan.stages, plan.group_m)
+    assert _lib.lib().i8l_launch_config(m, n, k, tuned, ctypes.byref(c)) == _lib.OK
+    return Config(c.bm, c.bn, c.bk, c.warps, c.stages, c.group_m)
+
+
+def test_every_shipped_entry_is_launched_at_its_own_token_count():
+    """No row of the tuned table is replaced by the launch rule at the token count that it was
+    measured at, and none is recorded slower than the library default there (beyond the few percent
+    that single timings of one table differ by: at most 3.2% in it)."""
+    tables = json.loads(kernel.TUNED_PATH.read_text())
+    rows = [(int(m), *map(int, kn.split("x")), row) for shapes in tables.values()
+            for kn, buckets in shapes.items() for m, row in buckets.items()]
+    assert len(rows) > 500
+    for m, k, n, row in rows:
+        cfg = Config(**row["config"])
+        assert _launched(m, n, k, cfg, m) == cfg, (m, k, n)
+        if "graph_us" in row:
+            assert row["graph_us"] <= 1.05 * row["default_us"], (m, k, n)
+
+
+def test_tuned_entry_is_kept_while_its_row_blocks_are():
+    """Past 128 tokens a tuned decode tile, and past 512 any tuned tile, is launched while the batch
+    makes the row blocks that it was tuned with, and not beyond; a split of K that its own user
+    tuned is never replaced at that token count."""
+    def kept(cfg, tuned, n, k):
+        return [m for m in range(tuned, 2 * tuned) if _launched(m, n, k, cfg, tuned) == cfg]
+
+    decode, stream = Config(16, 32, 128, 16, 4, 1), Config(32, 32, 256, 4, 1, 1)
+    assert kept(decode, 129, 1024, 2048) == list(range(129, 145))
+    assert kept(decode, 144, 1024, 2048) == [144]
+    assert kept(stream, 161, 1024, 2048) == list(range(161, 193))
+    assert kept(decode, 100, 1024, 2048) == list(range(100, 129))
+    ring = Config(256, 256, 128, 8, 10, 4)
+    assert kept(ring, 1000, 4096, 4096) == list(range(1000, 1025))
+    assert kept(ring, 500, 4096, 4096) == list(range(500, 513))
+    assert kept(Config(128, 128, 128, 4, 9, 4), 768, 4096, 14336) == [768]
+    split = Config(64, 64, 128, 4, 5, 2)
+    assert kept(split, 96, 4096, 14336) == list(range(96, 129))
+    assert kept(split, 64, 4096, 14336) == [64]
 
 
 def test_launch_config_takes_every_planned_shape():

@@ -5,11 +5,13 @@ capture.  The launch counter shows which path ran."""
 
 from __future__ import annotations
 
+from dataclasses import astuple
+
 import pytest
 import torch
 
 from helpers import ints, randn, say
-from int8_linear import _lib, kernel
+from int8_linear import Config, _lib, kernel
 from int8_linear import fused_quant as fq
 from int8_linear import vllm_patch
 from int8_linear.kernel import NotSupported, choose_config, w8a8_mm
@@ -48,12 +50,51 @@ def test_mm_binding_equals_ctypes_path(m, k, n, bias_dtype, ctypes_only):
     cfg = choose_config(m, n, k)
     assert fast().config_for(a.get_device(), m, n, k) == (cfg.bm, cfg.bn, cfg.bk, cfg.warps,
                                                           cfg.stages, cfg.group_m)
+    cfg = kernel.launch_config(m, n, k)
+    assert fast().launch_config_for(a.get_device(), m, n, k) == astuple(cfg)
     if (m, k, n) == (96, 14336, 4096):
-        assert cfg.stages == 5, cfg.name      # the shipped table splits K here
+        assert cfg.stages == 6 and cfg.group_m > 1, cfg.name  # the shipped table splits K here
     ctypes_only()
     ref = w8a8_mm(a, w.t(), sa, sb, torch.bfloat16, bias)
     torch.cuda.synchronize()
     assert torch.equal(got.view(torch.int16), ref.view(torch.int16))
+
+
+def test_binding_launches_what_launch_config_says():
+    """The binding's choice is kernel.launch_config's at every tuned bucket, between them and at
+    shapes without an entry: the plan, a replaced plan, a split of K."""
+    dev, seen = torch.cuda.current_device(), set()
+    w8a8_mm(ints((1, 2048), 1), ints((2048, 2048), 2).t(), torch.ones(1, device="cuda"),
+            torch.ones(1, device="cuda"))                # the first call hands the table over
+    shapes = [tuple(map(int, kn.split("x"))) for kn in kernel._device_table(dev)]
+    for k, n in shapes + [(13824, 5120), (2560, 9728), (4096, 5504), (2752, 4096), (64, 48)]:
+        for m in (1, 9, 16, 23, 64, 75, 96, 100, 128, 129, 136, 145, 161, 168, 200, 256, 257, 300,
+                  512, 513, 768, 777, 1024, 1025, 4096, 5000):
+            c, plan = kernel.launch_config(m, n, k), choose_config(m, n, k)
+            assert fast().launch_config_for(dev, m, n, k) == astuple(c), (m, n, k)
+            seen.add((c == plan, c.stages == 6 and c.group_m > 1))
+    assert {(True, False), (False, False), (False, True)} <= seen
+
+
+def test_binding_launches_a_tuned_split_of_k():
+    """A table whose entry is a stages-5 split (the shipped one holds none): the binding launches it
+    with a workspace of its own, with the unsplit tile's bits."""
+    m, k, n = 96, 14336, 4096
+    split = Config(64, 64, 128, 4, 5, 2)
+    a, w = ints((m, k), m), ints((n, k), n)
+    sa, sb = torch.rand((m, 1)).cuda() * 1e-2, torch.rand((n, 1)).cuda() * 1e-2
+    ref = w8a8_mm(a, w.t(), sa, sb, config=kernel.default_config(m, n, k))
+    dev = a.get_device()
+    say(f"binding mm split {split.name} m={m} k={k} n={n}")
+    fast().set_table(dev, [[k, n, m, *astuple(split)]])
+    try:
+        assert fast().launch_config_for(dev, m, n, k) == astuple(split)
+        before = fast().launches()
+        got = w8a8_mm(a, w.t(), sa, sb)
+        assert fast().launches() == before + 1
+    finally:
+        fast().set_table(dev, kernel._table_rows(dev))
+    assert torch.equal(got, ref)
 
 
 def test_mm_binding_declines_to_the_python_path():
