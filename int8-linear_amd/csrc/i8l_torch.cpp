@@ -113,8 +113,9 @@ py::object launch_config_for(int device, int64_t m, int64_t n, int64_t k) {
 
 // A fresh contiguous tensor on `like`'s device: at::empty's allocation (the caching allocator, under
 // a guard of the device) without its way through the dispatcher, which costs about as much again
-// on every output.  With a dispatch mode, a tracer or a function transform active, or a tensor
-// that is not a plain one, it goes through the dispatcher.
+// on every output.  With a dispatch mode, a tracer or a function transform active, a tensor that is
+// not a plain one, or new memory to be filled (deterministic algorithms), it goes through the
+// dispatcher.
 at::Tensor empty_like_on(const at::Tensor& like, at::IntArrayRef size, at::ScalarType dtype) {
   using c10::DispatchKey;
   static constexpr c10::DispatchKeySet kWatched(
@@ -125,7 +126,9 @@ at::Tensor empty_like_on(const at::Tensor& like, at::IntArrayRef size, at::Scala
        DispatchKey::FuncTorchVmapMode, DispatchKey::Batched, DispatchKey::VmapMode,
        DispatchKey::TESTING_ONLY_GenericMode, DispatchKey::DeferredInit, DispatchKey::Fake,
        DispatchKey::Tracer});
-  if ((c10::impl::tls_local_dispatch_key_set().included_ | like.key_set()).has_any(kWatched))
+  const at::Context& ctx = at::globalContext();
+  if ((c10::impl::tls_local_dispatch_key_set().included_ | like.key_set()).has_any(kWatched) ||
+      (ctx.deterministicAlgorithms() && ctx.deterministicFillUninitializedMemory()))
     return at::empty(size, like.options().dtype(dtype));
   return at::detail::empty_cuda(size, dtype, like.device(), std::nullopt);
 }

@@ -198,3 +198,34 @@ def test_outputs_under_a_dispatch_mode():
     assert sum("empty" in f for f in seen) == 2
     assert torch.equal(q, q0) and torch.equal(s, s0)
     assert q.is_contiguous() and not q.requires_grad and q.device == x.device
+
+
+def test_outputs_no_kernel_writes_are_filled_in_deterministic_mode():
+    """Under deterministic algorithms torch fills new memory: so it does the binding's outputs, which
+    shows where no kernel writes them (the scales of rows without columns)."""
+    say("binding outputs under deterministic algorithms")
+    x = torch.empty((300, 0), dtype=torch.bfloat16, device="cuda")
+    stale = torch.ones((300, 1), device="cuda")
+    del stale                               # its block is the next one of this size
+    torch.use_deterministic_algorithms(True)
+    try:
+        assert torch.utils.deterministic.fill_uninitialized_memory
+        q, s = fq.quant_per_token(x)
+        _, s2 = fq.silu_mul_quant(x, True, True)
+    finally:
+        torch.use_deterministic_algorithms(False)
+    assert q.shape == (300, 0) and bool(s.isnan().all()) and bool(s2.isnan().all())
+
+
+def test_outputs_under_a_tracer_and_inference_mode():
+    """torch.jit.trace records the binding's allocations; in inference mode they are inference
+    tensors."""
+    say("binding outputs under a tracer and in inference mode")
+    x = randn((5, 2048), 3)
+    q0, s0 = fq.quant_per_token(x)
+    graph = str(torch.jit.trace(lambda t: fq.quant_per_token(t), x, check_trace=False).graph)
+    assert graph.count("aten::empty") == 2, graph
+    with torch.inference_mode():
+        q, s = fq.quant_per_token(x)
+    assert q.is_inference() and s.is_inference()
+    assert torch.equal(q, q0) and torch.equal(s, s0)
