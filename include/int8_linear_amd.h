@@ -28,7 +28,7 @@ extern "C" {
 enum {
   I8L_OK = 0,
   I8L_UNSUPPORTED = 1, /* the kernels do not take this shape/dtype/config: caller falls back */
-  I8L_INVALID_ARG = 2, /* inconsistent shapes or sizes */
+  I8L_INVALID_ARG = 2, /* inconsistent shapes or sizes, or an operand that is NULL */
   I8L_HIP_ERROR = 3    /* a HIP runtime call failed (launch error, no device, ...) */
 };
 

@@ -6,6 +6,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <initializer_list>
 #include <type_traits>
 #include <stdint.h>
 
@@ -281,6 +282,16 @@ __device__ __forceinline__ void group_max_n(float (&v)[N]) {
 
 // ---------------------------------------------------------------- errors
 void set_error(const char* fmt, ...);
+// Whether every operand a launch would touch is there (a launch on a NULL one faults the GPU); an
+// error naming `who` otherwise.
+inline bool operands_ok(const char* who, std::initializer_list<const void*> operands) {
+  for (const void* p : operands)
+    if (!p) {
+      set_error("%s: an operand is NULL", who);
+      return false;
+    }
+  return true;
+}
 int hip_status(hipError_t e, const char* where);
 
 }  // namespace i8l

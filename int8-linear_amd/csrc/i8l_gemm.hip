@@ -423,6 +423,9 @@ int w8a8_mm(const int8_t* a, int64_t stride_am, int64_t stride_ak, const int8_t*
   int st = i8l_w8a8_mm_supported(M, N, K, &c);
   if (st != I8L_OK) return st;
   if (M == 0 || N == 0) return I8L_OK;
+  if (!operands_ok(who, {out}) || (K > 0 && !operands_ok(who, {a, b})) ||
+      (!raw && !operands_ok(who, {scale_a, scale_b})))
+    return I8L_INVALID_ARG;
 
   Epi e;
   e.sa = scale_a;
@@ -605,6 +608,7 @@ extern "C" int i8l_w8a8_mm_dynq(const void* x, int64_t ldx, int32_t act_dtype,
   const int st = i8l_w8a8_mm_dynq_supported(M, N, K, &c);
   if (st != I8L_OK) return st;
   if (M == 0 || N == 0) return I8L_OK;
+  if (!operands_ok("i8l_w8a8_mm_dynq", {x, b, scale_b, out})) return I8L_INVALID_ARG;
   const int osz = elt_size(out_dtype);
   const bool layout = stride_bk == 1 && aligned16(b) && stride_bn % 16 == 0 &&
                       stride_bn <= INT32_MAX / 32 && aligned16(x) && ldx % 8 == 0 &&
@@ -702,6 +706,7 @@ extern "C" int i8l_silu_mul_quant_mm(const void* gate_up, int64_t ldgu, int32_t 
   const int st = i8l_silu_mul_quant_mm_supported(M, N, K, &c);
   if (st != I8L_OK) return st;
   if (M == 0 || N == 0) return I8L_OK;
+  if (!operands_ok("i8l_silu_mul_quant_mm", {gate_up, b, scale_b, out})) return I8L_INVALID_ARG;
   const int osz = elt_size(out_dtype);
   const bool layout = stride_bk == 1 && aligned16(b) && stride_bn % 16 == 0 &&
                       stride_bn <= INT32_MAX / 32 && aligned16(gate_up) && ldgu % 8 == 0 &&
@@ -817,6 +822,7 @@ extern "C" int i8l_add_rmsnorm_quant_mm(const void* x, const void* residual, con
   const int st = i8l_add_rmsnorm_quant_mm_supported(M, N, K, &c);
   if (st != I8L_OK) return st;
   if (M == 0 || N == 0) return I8L_OK;
+  if (!operands_ok("i8l_add_rmsnorm_quant_mm", {b, scale_b, out})) return I8L_INVALID_ARG;
   const int osz = elt_size(out_dtype);
   const int64_t ncols = epilogue_act ? N / 2 : N;   // the output's columns
   const bool layout = stride_bk == 1 && aligned16(b) && stride_bn % 16 == 0 &&
@@ -927,6 +933,8 @@ extern "C" int i8l_w8a8_mm_silu_mul(const int8_t* a, int64_t stride_am, const in
   const int st = i8l_w8a8_mm_silu_mul_supported(M, N, K, &c);
   if (st != I8L_OK) return st;
   if (M == 0 || N == 0) return I8L_OK;
+  if (!operands_ok("i8l_w8a8_mm_silu_mul", {a, b, scale_a, scale_b, out}))
+    return I8L_INVALID_ARG;
   const bool layout = stride_bk == 1 && aligned16(b) && stride_bn % 16 == 0 &&
                       stride_bn <= INT32_MAX / 64 && aligned16(a) && stride_am % 16 == 0 &&
                       stride_am <= INT32_MAX / 128 && aligned16(out) && (stride_cm * 2) % 16 == 0 &&

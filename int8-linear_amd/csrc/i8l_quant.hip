@@ -639,6 +639,7 @@ extern "C" int i8l_add_rmsnorm_quant(const void* x, const void* residual, const 
     return I8L_UNSUPPORTED;
   }
   if (M == 0) return I8L_OK;
+  if (!operands_ok("add_rmsnorm_quant", {x, weight, q, scale})) return I8L_INVALID_ARG;
   const int h = (int)H;
   const bool vec = h % 8 == 0 && a16(x) && a16(weight) && a16(q) &&
                    (!residual || (a16(residual) && a16(residual_out)));
@@ -671,6 +672,7 @@ extern "C" int i8l_silu_mul_quant(const void* gate_up, int8_t* q, float* scale, 
     return I8L_UNSUPPORTED;
   }
   if (M == 0) return I8L_OK;
+  if (!operands_ok("silu_mul_quant", {gate_up, q, scale})) return I8L_INVALID_ARG;
   const int i = (int)I;
   const bool vec = i % 8 == 0 && a16(gate_up) && a16(q);
   const hipStream_t st = (hipStream_t)stream;
@@ -702,6 +704,7 @@ extern "C" int i8l_quant_per_token(const void* x, int64_t ldx, int8_t* q, float*
     return I8L_UNSUPPORTED;
   }
   if (M == 0) return I8L_OK;
+  if (!operands_ok("quant_per_token", {x, q, scale})) return I8L_INVALID_ARG;
   const int h = (int)H;
   const bool vec = h % 8 == 0 && ldx % 8 == 0 && a16(x) && a16(q);
   const Geom g = flat_geom(M, h, vec);

@@ -461,6 +461,35 @@ def test_tuner_candidate_sets(monkeypatch):
     assert tune.parse_ms("1,2,17") == [1, 2, 17]
 
 
+def test_every_entry_refuses_a_null_operand():
+    """An operand without memory (a NULL pointer, which is what a tensor wrapped by functionalize or a
+    fake tensor hands over) is an error before any launch, whichever it is."""
+    L, p = _lib.lib(), 4096
+    mm = [p, 64, 1, p, 1, 64, p, 1, p, 1, None, 0, p, 64, _lib.BF16, 4, 64, 64]
+    calls = [(L.i8l_w8a8_mm, mm + [None, None], (0, 3, 6, 8, 12)),
+             (L.i8l_w8a8_mm_ws, mm + [None, 0, None, None], (0, 3, 6, 8, 12)),
+             (L.i8l_w8a8_mm_noalloc, mm + [None, None], (0, 3, 6, 8, 12)),
+             (L.i8l_add_rmsnorm_quant, [p, p, p, 1e-6, p, p, p, 4, 64, _lib.BF16, _lib.BF16, 1, None],
+              (0, 2, 4, 5)),
+             (L.i8l_silu_mul_quant, [p, p, p, 4, 64, _lib.BF16, 1, 1, None], (0, 1, 2)),
+             (L.i8l_quant_per_token, [p, 64, p, p, 4, 64, _lib.BF16, 1, None], (0, 2, 3)),
+             (L.i8l_w8a8_mm_dynq, [p, 2048, _lib.BF16, 1, p, 1, 2048, p, 1, None, 0, p, 2048,
+                                   _lib.BF16, None, 4, 2048, 2048, None, None], (0, 4, 7, 11)),
+             (L.i8l_silu_mul_quant_mm, [p, 12288, _lib.BF16, 1, 1, p, 1, 6144, p, 1, None, 0, p,
+                                        2048, _lib.BF16, None, 1, 2048, 6144, None, None],
+              (0, 5, 8, 12)),
+             (L.i8l_add_rmsnorm_quant_mm, [p, p, p, 1e-6, _lib.BF16, 1, 0, p, p, 1, 2048, p, 4096,
+                                           None, 0, p, 4096, _lib.BF16, None, 4, 4096, 2048, None,
+                                           None], (0, 2, 8, 11, 15)),
+             (L.i8l_w8a8_mm_silu_mul, [p, 2048, p, 1, 2048, p, 1, p, 12288, None, 0, p, 6144, 1, 4,
+                                       12288, 2048, None, None], (0, 2, 5, 7, 11))]
+    for entry, args, operands in calls:
+        for i in operands:
+            bad = list(args)
+            bad[i] = None
+            assert entry(*bad) == _lib.INVALID_ARG, (entry.__name__, i, _lib.last_error())
+
+
 def _launched(m, n, k, plan, tuned):
     c = _lib.CConfig(plan.bm, plan.bn, plan.bk, plan.warps, plan.stages, plan.group_m)
     assert _lib.lib().i8l_launch_config(m, n, k, tuned, ctypes.byref(c)) == _lib.OK

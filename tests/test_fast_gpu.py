@@ -229,3 +229,31 @@ def test_outputs_under_a_tracer_and_inference_mode():
         q, s = fq.quant_per_token(x)
     assert q.is_inference() and s.is_inference()
     assert torch.equal(q, q0) and torch.equal(s, s0)
+
+
+def test_tensors_without_memory_are_refused(ctypes_only):
+    """vmap's wrapper has no data pointer and raises; functionalize's and a fake tensor's is 0, which
+    every entry refuses before it launches: with the binding and without."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    x = randn((3, 5, 2048), 4)
+    rows = x[0]
+    a, w, one = ints((5, 2048), 5), ints((2048, 2048), 6), torch.ones(1, device="cuda")
+
+    def refused():
+        with pytest.raises(RuntimeError):
+            torch.func.vmap(lambda t: fq.quant_per_token(t)[0])(x)
+        with pytest.raises(ValueError):
+            torch.func.functionalize(lambda t: fq.quant_per_token(t)[0])(rows)
+        with pytest.raises(ValueError):
+            torch.func.functionalize(lambda t: w8a8_mm(t, w.t(), one, one))(a)
+        with FakeTensorMode() as mode, pytest.raises(ValueError):
+            fq.silu_mul_quant(mode.from_tensor(rows), True, True)
+
+    say("tensors without memory, binding")
+    before = fast().launches()
+    refused()
+    assert fast().launches() == before
+    ctypes_only()
+    say("tensors without memory, ctypes")
+    refused()
