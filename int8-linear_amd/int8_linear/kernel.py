@@ -143,9 +143,9 @@ def choose_config(m: int, n: int, k: int) -> Config:
 
 def launch_config(m: int, n: int, k: int, planned: Config | None = None) -> Config:
     """The config a call without an explicit one launches (i8l_launch_config): choose_config's
-    (or `planned`, as one tuned for a single token), or the tile with the least modelled time where
-    no tuned entry lies close below M.  A tuned entry is always launched at its own token count."""
-    bucket = 1 if planned is not None else tuned_bucket(m, n, k)
+    (`planned`, where the caller has it at hand), or the tile with the least modelled time where no
+    tuned entry lies close below M.  A tuned entry is always launched at its own token count."""
+    bucket = tuned_bucket(m, n, k) if torch.cuda.is_available() else 0
     p = planned or choose_config(m, n, k)
     c = _lib.CConfig(p.bm, p.bn, p.bk, p.warps, p.stages, p.group_m)
     _lib.check(_lib.lib().i8l_launch_config(m, n, k, bucket, c), NotSupported)

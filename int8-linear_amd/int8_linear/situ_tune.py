@@ -6,8 +6,8 @@ mispredicted it (AshrithaG/int8-linear, bench/situ_tune.py:1-34 and 214-255; REA
 decode step, where 28 layers with their own weights run with the quantizers between them.
 
 For a batch of m tokens this makes one pass over the four linears of the stand-in
-(int8_linear.standin): each linear tries its current configuration (the tuned table's or the
-library default's), the library default and the `top` fastest configurations of an
+(int8_linear.standin): each linear tries its current configuration (what a call without one
+launches), the library default and the `top` fastest configurations of an
 isolated sweep of that shape, with the other three fixed, and keeps whichever makes the
 stand-in's step (one HIP graph of all 28 layers) fastest.  The chosen set is then timed
 against the starting set in alternating fresh captures, and kept only if it is at least
@@ -42,7 +42,7 @@ import torch
 
 from int8_linear import fused_quant as fq
 from int8_linear import tune
-from int8_linear.kernel import Config, choose_config, default_config, supported, w8a8_mm
+from int8_linear.kernel import Config, default_config, launch_config, supported, w8a8_mm
 from int8_linear.operands import operands, seed_of
 from int8_linear.standin import HIDDEN, INTER, SHAPES, DecoderStandIn, per_layer_us
 
@@ -158,8 +158,8 @@ def situ_tune(m: int, layers: int = 28, top: int = 4, rounds: int = 5, windows: 
     "trials", "confirm_us" (start/chosen, when they differ), "kept"}."""
     stack = stack or DecoderStandIn(m, layers=layers, device=device)
     kinds = kernels(stack)
-    # w8a8_mm linears start from the table's choice, the folded kernels from their default
-    start = {name: choose_config(m, n, k) if kinds[name] == "mm" else None
+    # w8a8_mm linears start from what a call launches, the folded kernels from their default
+    start = {name: launch_config(m, n, k) if kinds[name] == "mm" else None
              for name, (k, n) in SHAPES.items()}
     current = dict(start)
     trials = []

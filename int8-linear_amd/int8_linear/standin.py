@@ -58,7 +58,7 @@ class DecoderStandIn:
         g = torch.Generator(device=generator_device).manual_seed(seed)
         dev = torch.device(device)
         self.m = m
-        # per-linear configurations ({name: Config}); a linear not named takes choose_config
+        # per-linear configurations ({name: Config}); a linear not named takes launch_config's
         self.configs: dict = {}
         # the same for the norm-folded linears ({name: Config}, else the library's choice)
         self.norm_configs: dict = {}

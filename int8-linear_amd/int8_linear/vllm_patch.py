@@ -28,7 +28,8 @@ from typing import Optional
 
 import torch
 
-from int8_linear.kernel import NotSupported, choose_config, tuned_config, w8a8_mm
+from int8_linear.kernel import (NotSupported, choose_config, launch_config, tuned_config,
+                                w8a8_mm)
 
 CALLS = 0
 FALLBACKS = 0
@@ -38,11 +39,12 @@ _vllm_triton_scaled_mm = None
 
 
 def _note(m: int, k: int, n: int) -> None:
-    """Count the call and record which configuration (M, K, N) runs with."""
+    """Count the call and record which configuration (M, K, N) runs with: the one that is launched,
+    not the plan it is made of."""
     global CALLS
     CALLS += 1
     if (m, k, n) not in CONFIGS:
-        CONFIGS[(m, k, n)] = choose_config(m, n, k).name
+        CONFIGS[(m, k, n)] = launch_config(m, n, k, choose_config(m, n, k)).name
 
 
 def _run(a_q: torch.Tensor, b_q: torch.Tensor, scale_a: torch.Tensor, scale_b: torch.Tensor,

@@ -176,6 +176,19 @@ def test_vllm_entry_uses_the_binding_and_records_configs():
     assert torch.equal(out, kernel.w8a8_mm(a, w.t(), sa, sb, config=choose_config(4, 2048, 2048)))
 
 
+@pytest.mark.parametrize("m,k,n", [(100, 13824, 5120), (600, 2560, 9728)])
+def test_vllm_entry_records_what_is_launched(m, k, n):
+    """CONFIGS holds the launched configuration where it is not the plan."""
+    a, w = ints((m, k), 8), ints((n, k), 9)
+    sa, sb = torch.rand((m, 1), device="cuda"), torch.rand((n, 1), device="cuda")
+    vllm_patch.CONFIGS.pop((m, k, n), None)
+    out = vllm_patch.scaled_mm(a, w.t(), sa, sb, torch.bfloat16)
+    launched = kernel.launch_config(m, n, k)
+    assert launched != choose_config(m, n, k)
+    assert vllm_patch.CONFIGS[(m, k, n)] == launched.name
+    assert torch.equal(out, kernel.w8a8_mm(a, w.t(), sa, sb, config=launched))
+
+
 def test_outputs_under_a_dispatch_mode():
     """The binding allocates its outputs past the dispatcher, except where a dispatch mode or a
     function transform is active: a mode then sees the allocations, and the outputs are the same."""
