@@ -112,7 +112,8 @@ gemm_phased(const int8_t* __restrict__ A, int64_t lda, const int8_t* __restrict_
   const int8_t *pA, *pB;   // the K position being requested, in the tile being requested
   auto tile_at = [&](int tile, int64_t& mt, int64_t& nt) {
     int pid_m, pid_n;
-    staged_tile(tile, tiles, num_pid_m, num_pid_n, group_m, pid_m, pid_n);
+    staged_tile(tiles % 8 == 0 ? tile : xcd_order(tile, tiles), tiles, num_pid_m, num_pid_n, group_m,
+                pid_m, pid_n);
     mt = (int64_t)pid_m * BM;
     nt = (int64_t)pid_n * BN;
   };

@@ -85,6 +85,17 @@ __device__ __forceinline__ void staged_tile(int pid, int npid, int num_pid_m, in
   pid_n = (pid % in_group) / gsize;
 }
 
+// Position `pid` of `npid` in the order staged_tile makes of a multiple of 8, for any other count:
+// consecutive positions go to one XCD, the first npid % 8 XCDs taking one more.  The phased tiles
+// need it: without, an operand's rows are fetched into every XCD's L2, and 222 tiles of 128 x 256
+// (331 tokens, 3584 -> 18944) took 42.3 us where the ring of that size takes 38; with it 32.3.
+// 1536 -> 8960 at 2500 tokens (128 x 256) 62.9 -> 45.9, 2560 -> 9728 at 300 (128 x 128) 22.6 ->
+// 15.9, 1792 -> 9792 at 1543 (128 x 192) 55.8 -> 51.1.
+__device__ __forceinline__ int xcd_order(int pid, int npid) {
+  const int x = pid % 8;
+  return x * (npid / 8) + min(x, npid % 8) + pid / 8;
+}
+
 typedef __attribute__((address_space(3))) int8_t lds_i8;
 
 // s_waitcnt with vmcnt = N and the LGKM / EXP counters left unconstrained (gfx9 encoding:

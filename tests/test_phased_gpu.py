@@ -46,6 +46,20 @@ def test_several_tiles_a_workgroup(config):
 
 
 @pytest.mark.parametrize("config", TILES, ids=ids)
+@pytest.mark.parametrize("tiles_m,tiles_n", [(1, 1), (1, 7), (3, 3), (5, 3), (9, 29), (19, 27)])
+def test_tile_counts_that_eight_does_not_divide(config, tiles_m, tiles_n):
+    """Every tile is computed once, whatever number of them the 8 XCDs share: fewer than 8, one more
+    or less than a multiple, more than the workgroups."""
+    m, n, k = tiles_m * config.bm - 3, tiles_n * config.bn, 512
+    assert tiles_m * tiles_n % 8
+    say(f"phased {config.name} {tiles_m} x {tiles_n} tiles")
+    a, w = ints((m, k), tiles_m), ints((n, k), tiles_n)
+    one = torch.ones(1, device="cuda")
+    got = w8a8_mm(a, w.t(), one, one, raw=True, config=config)
+    assert np.array_equal(np_(got), o.gemm_i32(np_(a), np_(w)))
+
+
+@pytest.mark.parametrize("config", TILES, ids=ids)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_every_bias_and_scale(config, dtype):
     code = {torch.bfloat16: o.BF16, torch.float16: o.F16, torch.float32: o.F32}
