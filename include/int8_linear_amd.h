@@ -56,7 +56,7 @@ enum {
  *                of 16) token rows a workgroup (decode on long K; splits K as stages 5 does);
  *                2 LDS staged through registers, 3..8 with bm >= 128 and bn >= 128 a ring of
  *                that many direct-to-LDS buffers, 9 persistent macro tiles of 4 waves whose
- *                steps are cut into four phases (K a multiple of 2 * bk, from 4 * bk on), >= 10
+ *                128-byte steps are cut into four phases (K a multiple of 256, from 512 on), >= 10
  *                a ring of stages - 8 buffers (2: a double buffer) with fragment reads
  *                overlapped with the MFMAs (prefill)
  *   group_m    : rows of tiles walked together for L2 reuse (1 = row-major order); stages 3

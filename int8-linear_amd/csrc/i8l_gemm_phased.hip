@@ -384,16 +384,15 @@ gemm_phased(const int8_t* __restrict__ A, int64_t lda, const int8_t* __restrict_
 
 // ------------------------------------------------------------------ host side
 struct PhasedTile {
-  int bm, bn, bk;
+  int bm, bn;
 };
-constexpr PhasedTile kPhased[] = {{256, 256, 128}, {256, 192, 128}, {256, 128, 128},
-                                  {128, 256, 128}, {128, 192, 128}, {128, 128, 128},
-                                  {128, 128, 256}};
+constexpr PhasedTile kPhased[] = {{256, 256}, {256, 192}, {256, 128},
+                                  {128, 256}, {128, 192}, {128, 128}};
 
 int phased_index(const i8l_config& c, int64_t K) {
-  if (c.stages != kPhasedStages || c.warps != 4 || c.group_m < 1) return -1;
+  if (c.stages != kPhasedStages || c.warps != 4 || c.bk != 128 || c.group_m < 1) return -1;
   for (int i = 0; i < (int)(sizeof(kPhased) / sizeof(kPhased[0])); ++i)
-    if (kPhased[i].bm == c.bm && kPhased[i].bn == c.bn && kPhased[i].bk == c.bk)
+    if (kPhased[i].bm == c.bm && kPhased[i].bn == c.bn)
       // whole pairs of steps, the first and the last apart
       return K % (2 * c.bk) == 0 && K >= 4 * c.bk ? i : -1;
   return -1;
@@ -442,7 +441,6 @@ hipError_t launch_phased(int idx, const i8l_config& c, const int8_t* a, int64_t 
     case 3: return launch_phased_t<1, 2, 2, 128>(a, lda, b, ldb, e, K, c.group_m, st);
     case 4: return launch_phased_t<1, 2, 1, 128>(a, lda, b, ldb, e, K, c.group_m, st);
     case 5: return launch_phased_t<1, 1, 1, 128>(a, lda, b, ldb, e, K, c.group_m, st);
-    case 6: return launch_phased_t<1, 1, 1, 256>(a, lda, b, ldb, e, K, c.group_m, st);
   }
   return hipErrorInvalidValue;
 }

@@ -532,6 +532,14 @@ def test_tuned_entry_is_kept_while_its_row_blocks_are():
     assert kept(split, 64, 4096, 14336) == [64]
 
 
+def test_every_phased_tile_is_a_candidate():
+    """The library takes no phased tile that the tuner (and the GPU tests, by its list) does not."""
+    from int8_linear import tune
+    built = [(bm, bn) for bm in range(64, 513, 64) for bn in range(64, 513, 64) for bk in (64, 128, 256)
+             if kernel.supported(1024, 64 * 45 * 7 * 16, 4096, Config(bm, bn, bk, 4, tune.PHASED, 4))]
+    assert sorted(built) == sorted(tune.PHASED_TILES)
+
+
 def test_launch_config_takes_every_planned_shape():
     """What a call launches is built and takes the shape whatever was planned; a decode plan on
     short K is launched as it is up to 128 tokens, and so is a tuned one, and a tuned macro tile up
