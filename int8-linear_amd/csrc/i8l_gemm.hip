@@ -184,21 +184,30 @@ void default_config(int64_t M, int64_t N, int64_t K, i8l_config* c) {
 // A tile's `rounds` is 0.7 times the whole rounds its workgroups make over the slots (compute units
 // times workgroups a unit) plus 0.3 times the exact ratio (a round of which a part is idle is as
 // long, but the clock is higher); where two fit a unit, one alone takes `alone` of their time.  The
-// numbers of each tile are fitted to its measured times (rms error 5-15%) on MI355X.
-//  * From 129 tokens on (33 where the plan is a macro tile already): 33 weight shapes, K
-//    1024-28672, N 1024-57344, 33-5000 tokens.  The pick takes 1.007x the fastest tile's time on
-//    the geometric mean, 1.006x over eight of the shapes left out of the fit, where the plan takes
-//    1.08-1.13x, and 1.2-1.3x at tuned shapes between their buckets (512, 1024, 2048, 4096).  So a
-//    tuned macro tile is kept up to 512 tokens, where buckets lie 8-16 tokens apart, and a tuned
-//    decode tile up to 128.  Beyond, an entry is kept while the batch makes the row blocks that it
-//    was measured with, so at its own token count always: 2048x1024 at 144 tokens 5.5 us in 9
-//    blocks of 16 rows, 8.1 at 145 in 10, the pick 7.2.  The phased tiles (K a multiple
-//    of 256, from 512) beat the ring of their own size at all of these points but two, so the
-//    larger rings serve the other K.
-//  * 33-128 tokens, no tuned entry: 19 shapes, K 1024-28672, N 1536-18944, where the plan takes
-//    1.2-1.44x the fastest tile's time and the pick 1.03x.  Up to K = 2048 the plan's single-step
-//    tiles are the better (or the equal), unless it fell back to streaming.  The shared ring is the
-//    pick on long K, where it is up to 2.1x faster than the plan.
+// numbers of each tile are fitted to its measured times (rms error 4-9%) on MI355X, and a ring whose
+// tiles 8 does not divide, so that they get no XCD order, is priced 4% higher.  `python -m
+// int8_linear.tune --launch-rule` times plan, pick and every tile and fits the numbers again.
+//  * From 129 tokens on (33 where the plan is a macro tile already): 461 cases of 32 weight shapes, K
+//    128-18944, N 512-18944, 129-4096 tokens.  The pick takes 1.003x the fastest tile's time on the
+//    geometric mean and at worst 1.04x the plan's, the plan 1.09x (fitted on every other shape, over
+//    the rest: 1.004x from K = 1024, 1.02x below).  In 1273 further cases where it differs from the
+//    plan (random shapes and batches from 17 tokens on) it takes 0.77x the plan's time, and over
+//    1.03x in 24.  At tuned shapes between their buckets (512, 1024, 2048, 4096) the plan takes
+//    1.2-1.3x.  So a tuned macro tile is kept up to 512 tokens, where buckets lie 8-16 tokens apart,
+//    and a tuned decode tile up to 128.  Beyond, an entry is kept while the batch makes the row
+//    blocks that it was measured with, so at its own token count always: 2048x1024 at 144 tokens 5.5
+//    us in 9 blocks of 16 rows, 8.1 at 145 in 10, the pick 7.2.  The phased tiles (K a multiple of
+//    256, from 512) beat the ring of their own size at nearly all of these points, so the larger
+//    rings serve the other K.
+//  * 33-128 tokens, no tuned entry: 23 shapes, K 512-18944, N 1024-18944, where the plan takes 1.36x
+//    the fastest tile's time and the pick 1.012x, nowhere more than the plan's.  Up to K = 2048 the
+//    plan's single-step tiles are the better (or the equal), unless it fell back to streaming.
+//    Streaming in turn, up to 64 tokens, in one round of workgroups and 8 steps a wave, beats every
+//    tile (1792x4096 at 33 tokens 6.1 us, the pick 6.9; 768x3072 4.3, 4.9; in two rounds it loses,
+//    1280x5120 7.6, 6.1, and with 11 steps, 1408x960 6.2, 5.5; up to 32 tokens it wins with 9 and
+//    11, 2304x4096 5.7, 6.6 and 2816x3776 6.8, 7.5, and loses with 17).  The shared ring is the pick
+//    on long K, where it is up to 2.1x faster than the plan.  The 64x64 ring takes 4% longer on one
+//    or two row blocks than its numbers say.
 //  * 17-32 tokens, no tuned entry, K above 2048: the plan's 32x32 tiles are within 4% of the
 //    fastest (7168x7168 at 23 tokens: 12.1 us, the pick 13.0), so only its narrower ones, which
 //    read A once for every 8 or 16 columns, are replaced (4096x5504: 11.7 -> 7.4 us).
@@ -227,27 +236,29 @@ static float modelled_us(const ModelTile& t, int64_t M, int64_t N, int64_t K, in
 static void launch_config(int64_t M, int64_t N, int64_t K, int64_t tuned, bool split,
                           i8l_config* c) {
   static constexpr ModelTile kMacro[] = {
-      {256, 256, 4, kPhasedStages, 4, 1, 1.0f, 0.0f, 10.75f, 9.87f},
-      {256, 192, 4, kPhasedStages, 4, 1, 1.0f, 0.6f, 8.85f, 7.04f},
-      {256, 128, 4, kPhasedStages, 4, 1, 1.0f, 2.05f, 6.74f, 2.9f},
-      {128, 256, 4, kPhasedStages, 8, 1, 1.0f, 3.82f, 7.58f, 0.44f},
-      {128, 192, 4, kPhasedStages, 8, 1, 1.0f, 4.14f, 6.15f, 0.73f},
-      {128, 128, 4, kPhasedStages, 8, 2, 0.6f, 1.94f, 8.37f, 1.47f},
-      {64, 64, 4, 4 + kPipelined, 8, 1, 1.0f, 4.19f, 1.92f, 0.01f},
-      {128, 64, 4, 4 + kPipelined, 8, 1, 1.0f, 2.42f, 3.05f, 1.92f},
-      {64, 128, 4, 4 + kPipelined, 8, 1, 1.0f, 2.89f, 3.33f, 1.6f},
-      {64, 256, 8, 3 + kPipelined, 8, 1, 1.0f, 3.67f, 6.07f, 0.4f},
-      {128, 128, 4, 4 + kPipelined, 8, 1, 1.0f, 3.07f, 4.73f, 2.72f},
-      {256, 128, 8, 3 + kPipelined, 8, 1, 1.0f, 1.24f, 7.66f, 4.8f},
-      {128, 256, 8, 3 + kPipelined, 8, 1, 1.0f, 3.0f, 8.19f, 2.94f},
-      {256, 192, 8, 2 + kPipelined, 4, 1, 1.0f, 4.56f, 10.72f, 3.31f},
-      {256, 256, 8, 2 + kPipelined, 4, 1, 1.0f, 2.21f, 13.15f, 4.96f}};
-  static constexpr ModelTile kDecode[] = {{64, 32, 4, 3, 3, 1, 1.0f, 1.71f, 1.65f, 1.83f},
-                                          {32, 32, 4, 3, 3, 1, 1.0f, 1.46f, 1.28f, 1.34f},
-                                          {32, 64, 4, 3, 3, 1, 1.0f, 1.61f, 2.03f, 1.98f},
-                                          {32, 16, 4, 3, 3, 2, 0.5f, 2.32f, 1.72f, 0.3f},
-                                          {16, 32, 4, 3, 4, 1, 1.0f, 0.5f, 1.06f, 1.53f},
-                                          {16, 16, 4, 3, 4, 2, 0.5f, 1.78f, 1.34f, 0.29f}};
+      {256, 256, 4, kPhasedStages, 4, 1, 1.0f, 2.95f, 10.24f, 7.31f},
+      {256, 192, 4, kPhasedStages, 4, 1, 1.0f, 2.21f, 8.25f, 6.58f},
+      {256, 128, 4, kPhasedStages, 4, 1, 1.0f, 2.62f, 6.29f, 3.51f},
+      {128, 256, 4, kPhasedStages, 8, 1, 1.0f, 3.74f, 7.17f, 2.26f},
+      {128, 192, 4, kPhasedStages, 8, 1, 1.0f, 3.48f, 5.83f, 1.72f},
+      {128, 128, 4, kPhasedStages, 8, 2, 0.6f, 2.39f, 7.71f, 3.39f},
+      {64, 64, 4, 4 + kPipelined, 8, 2, 0.6f, 2.61f, 3.46f, 1.92f},
+      {128, 64, 4, 4 + kPipelined, 8, 1, 1.0f, 1.92f, 2.86f, 2.78f},
+      {64, 128, 4, 4 + kPipelined, 8, 1, 1.0f, 2.26f, 3.21f, 2.58f},
+      {64, 256, 8, 3 + kPipelined, 8, 1, 1.0f, 3.0f, 5.8f, 2.27f},
+      {128, 128, 4, 4 + kPipelined, 8, 1, 1.0f, 2.57f, 4.52f, 3.83f},
+      {256, 128, 8, 3 + kPipelined, 8, 1, 1.0f, 1.58f, 7.31f, 5.28f},
+      {128, 256, 8, 3 + kPipelined, 8, 1, 1.0f, 2.36f, 7.79f, 4.62f},
+      {256, 192, 8, 2 + kPipelined, 4, 1, 1.0f, 3.9f, 10.78f, 3.99f},
+      {256, 256, 8, 2 + kPipelined, 4, 1, 1.0f, 1.01f, 12.53f, 8.62f}};
+  static constexpr ModelTile kDecode[] = {{64, 32, 4, 3, 3, 1, 1.0f, 2.05f, 1.57f, 1.49f},
+                                          {32, 32, 4, 3, 3, 1, 1.0f, 1.45f, 1.2f, 1.38f},
+                                          {32, 64, 4, 3, 3, 1, 1.0f, 1.62f, 1.97f, 1.84f},
+                                          {32, 16, 4, 3, 3, 1, 1.0f, 2.13f, 0.8f, 0.3f},
+                                          {16, 32, 4, 3, 4, 1, 1.0f, 0.47f, 0.93f, 1.87f},
+                                          {16, 16, 4, 3, 4, 2, 0.6f, 1.06f, 1.19f, 0.83f}};
+  // the plan's own tile where K is a multiple of 1024 (256-byte steps)
+  static constexpr ModelTile kPlanned{32, 32, 4, 3, 1, 2, 0.4f, 2.58f, 2.76f, -0.08f};
   static constexpr ModelTile kSixteen[] = {{16, 32, 4, 3, 3, 2, 0.5f, 2.28f, 2.13f, 0.91f},
                                            {16, 16, 4, 3, 4, 2, 0.5f, 2.16f, 1.17f, 0.84f},
                                            {16, 64, 4, 3, 4, 1, 1.0f, 0.6f, 1.85f, 2.93f}};
@@ -265,8 +276,8 @@ static void launch_config(int64_t M, int64_t N, int64_t K, int64_t tuned, bool s
       const int64_t wgs = N / 64 * z;
       const float rounds = 0.7f * (float)((wgs + cus - 1) / cus) + 0.3f * (float)wgs / (float)cus;
       const float steps = (float)(K / 128) / (float)z;
-      consider(2.15f + rounds * (steps * (0.2541f + 0.0023f * (float)ring_bm) + 1.82f) +
-                   (z > 1 ? 1.19f + 1.21e-6f * (float)z * (float)M * (float)N : 0.0f), cand);
+      consider(2.49f + rounds * (steps * (0.2172f + 0.0028f * (float)ring_bm) + 1.51f) +
+                   (z > 1 ? 0.96f + 1.19e-6f * (float)z * (float)M * (float)N : 0.0f), cand);
     }
   };
   auto blocks = [&](int64_t m) { return (m + c->bm - 1) / c->bm; };
@@ -281,10 +292,13 @@ static void launch_config(int64_t M, int64_t N, int64_t K, int64_t tuned, bool s
     return;
   }
   if (K % 128 != 0 || N % 64 != 0) return;
+  const bool streams = c->stages == 1;
+  const int64_t few_steps = M <= 32 ? 12 : 8;
+  if (streams && M <= 64 && K >= 512 && K <= few_steps * c->bk && N / c->bn <= cus) return;
   const bool half = M <= 16 && c->bm > 16;      // a decode plan, half of its rows idle
   const bool narrow = M > 16 && c->bn < 32;
   const bool decode = !tuned && M <= 128 &&
-                      (M > 32 ? K > 2048 || c->stages == 1 : narrow && K > 2048);
+                      (M > 32 ? K > 2048 || streams : narrow && K > 2048);
   const bool sixteen = !tuned && !macro && half && K > 2048 && N < 24576;
   if (M <= 128 && !macro && !decode && !sixteen) return;
   const bool phased = K % 256 == 0 && K >= 512;
@@ -295,13 +309,18 @@ static void launch_config(int64_t M, int64_t N, int64_t K, int64_t tuned, bool s
     }
     return;
   }
+  const i8l_config plan = *c;
   for (const auto& t : kMacro) {
     const bool ph = t.stages == kPhasedStages;
     if (N % t.bn != 0 || (phased ? !ph && t.bm * t.bn >= 128 * 128 && t.bm > 64 : ph)) continue;
-    consider(modelled_us(t, M, N, K, cus),
+    const bool ragged = !ph && (M + t.bm - 1) / t.bm * (N / t.bn) % 8 != 0;
+    const bool few = t.bm == 64 && t.bn == 64 && M <= 128;
+    consider(modelled_us(t, M, N, K, cus) * (ragged || few ? 1.04f : 1.0f),
              i8l_config{t.bm, t.bn, 128, t.warps, t.stages, t.group_m});
   }
   if (!decode) return;
+  if (plan.bm == 32 && plan.bn == 32 && plan.bk == 256 && plan.stages == 3)
+    consider(modelled_us(kPlanned, M, N, K, cus), plan);
   for (const auto& t : kDecode) {
     const i8l_config cand{t.bm, t.bn, 128, t.warps, t.stages, t.group_m};
     if (wlds_ok(cand, K)) consider(modelled_us(t, M, N, K, cus), cand);

@@ -7,10 +7,13 @@ reference's sweep and merge are bench/bench_linear.py:213-227, 385-389).
     python -m int8_linear.tune --shapes llama-3-8b --m 512,1024,2048,4096 --merge
     python -m int8_linear.tune --shapes qwen3-1.7b-vllm --m capture --merge
     python -m int8_linear.tune --ring-costs [--kn 8192x8192,...] [--m 48,96,...]
+    python -m int8_linear.tune --launch-rule [--kn 8192x8192,...] [--m 48,96,...]
 
 `--ring-costs` times the overlapped-ring tiles the library default chooses among (their
 per-wave costs are the constants of that rule) and checks the default's pick against the
-fastest of them.  `--m capture` is vLLM's CUDA-graph batch sizes (1, 2, 4, 8 to 248 by 8, 256 to 512 by 16)
+fastest of them.  `--launch-rule` does the same for i8l_launch_config, which a call without a
+tuned entry launches: plan, launched tile and every tile the rule prices, and the rule's
+constants fitted to those times.  `--m capture` is vLLM's CUDA-graph batch sizes (1, 2, 4, 8 to 248 by 8, 256 to 512 by 16)
 plus three prefill sizes, the M values a served decode step is padded to (the reference's
 tools/run_e2e_vm.sh:60-67).
 
@@ -373,12 +376,150 @@ def ring_costs(shapes: str = RING_SHAPES, ms: str = RING_MS, log=print) -> dict:
     return out
 
 
+# (bm, bn, warps, stages, group_m, workgroups a compute unit) of the tiles i8l_launch_config
+# prices (csrc/i8l_gemm.hip; with the default's 32x32x256); the shared ring is priced by a
+# formula of its own there
+MODEL_MACRO = [(256, 256, 4, PHASED, 4, 1), (256, 192, 4, PHASED, 4, 1), (256, 128, 4, PHASED, 4, 1),
+               (128, 256, 4, PHASED, 8, 1), (128, 192, 4, PHASED, 8, 1), (128, 128, 4, PHASED, 8, 2),
+               *((bm, bn, w, st, g, 2 if bm == bn == 64 else 1) for bm, bn, _, w, st, g in RING)]
+MODEL_DECODE = [(64, 32, 4, 3, 3, 1), (32, 32, 4, 3, 3, 1), (32, 64, 4, 3, 3, 1),
+                (32, 16, 4, 3, 3, 1), (16, 32, 4, 3, 4, 1), (16, 16, 4, 3, 4, 2)]
+MODEL_SIXTEEN = [(16, 32, 4, 3, 3, 2), (16, 16, 4, 3, 4, 2), (16, 64, 4, 3, 4, 1)]
+RULE_SHAPES = ("384x768,512x4096,768x3072,1024x4096,1280x5120,1536x8960,1792x4096,2048x2048,"
+               "2048x12288,2560x9728,3584x4608,3584x18944,4096x1536,4096x5504,4096x6144,5120x5120,"
+               "5120x7680,6144x2048,8192x10240,13824x5120,18944x3584")
+RULE_MS = "1,8,16,23,33,48,64,75,100,128,129,200,300,512,777,1024,1500,2048,4096"
+
+
+def rule_rounds(tile: tuple, alone: float, m: int, n: int, cus: int) -> float:
+    """The rounds i8l_launch_config prices a tile at (see the comment there)."""
+    bm, bn, per_cu = tile[0], tile[1], tile[5]
+    wgs, slots = -(-m // bm) * (n // bn), per_cu * cus
+    rest = wgs % slots
+    last = 0.0 if rest == 0 else alone if per_cu > 1 and rest <= cus else 1.0
+    return 0.7 * (wgs // slots + last) + 0.3 * wgs / slots
+
+
+def _relative_fit(rows: list[list[float]], us: list[float]) -> tuple[list[float], float]:
+    """Coefficients of the columns of `rows` with the least squared relative error against the
+    times, and that error's root mean square."""
+    t = torch.tensor(us, dtype=torch.float64)
+    x = torch.tensor(rows, dtype=torch.float64) / t[:, None]
+    c = torch.linalg.lstsq(x, torch.ones_like(t)[:, None]).solution[:, 0]
+    return c.tolist(), float(((x @ c - 1) ** 2).mean().sqrt())
+
+
+def fit_tile(tile: tuple, points: list, cus: int) -> dict:
+    """One tile's numbers for the rule (alone, fixed, step, turn), fitted to its measured times:
+    points of (k, n, m, us)."""
+    best = None
+    # (a ring without an XCD order is priced 4% higher)
+    points = [(k, n, m, us / (1.04 if tile[3] > PHASED and -(-m // tile[0]) * (n // tile[1]) % 8
+                              else 1.0)) for k, n, m, us in points]
+    for alone in ((0.4, 0.5, 0.6, 0.7, 0.8, 0.9, 1.0) if tile[5] > 1 else (1.0,)):
+        r = [rule_rounds(tile, alone, m, n, cus) for _, n, m, _ in points]
+        c, rms = _relative_fit([[1.0, x * p[0] * 1e-3, x] for x, p in zip(r, points)],
+                               [p[3] for p in points])
+        if best is None or rms < best["rms"]:
+            best = {"alone": alone, "fixed": c[0], "step": c[1], "turn": c[2], "rms": rms,
+                    "points": len(points)}
+    return {key: round(v, 4) for key, v in best.items()}
+
+
+def fit_shared_ring(points: list, cus: int) -> dict:
+    """The same for the shared ring: points of (k, n, m, us, token rows, parts of K)."""
+    rows = []
+    for k, n, m, _, bm, z in points:
+        wgs = n // 64 * z
+        r = 0.7 * -(-wgs // cus) + 0.3 * wgs / cus
+        s = r * (k / 128) / z
+        rows.append([1.0, s, s * bm, r, float(z > 1), z * m * n * (z > 1) * 1e-6])
+    c, rms = _relative_fit(rows, [p[3] for p in points])
+    names = ("fixed", "step", "step_per_row", "turn", "split", "split_per_million")
+    return {**{key: round(v, 4) for key, v in zip(names, c)}, "rms": round(rms, 4),
+            "points": len(points)}
+
+
+def launch_rule(shapes: str = RULE_SHAPES, ms: str = RULE_MS, log=print) -> dict:
+    """Time the tiles i8l_launch_config chooses among for calls without a tuned entry, beside the
+    plan (i8l_default_config) and what it launches.
+
+    Logged: one line a case with the plan's, the launched tile's and the fastest tile's times;
+    then, over the cases, how far the plan and the launched tile are from the fastest, and the
+    cases where the launched tile is over 2% slower than the plan; last, each tile's constants
+    fitted to these times, of the batches it is priced for from 17 tokens on (those of the rule,
+    csrc/i8l_gemm.hip, are one such fit: the macro tiles' over the batches past 128)."""
+    import math
+
+    from int8_linear import _lib
+    dev = torch.device("cuda:0")
+    cus = torch.cuda.get_device_properties(dev).multi_processor_count
+    log(f"{torch.cuda.get_device_name(dev)}: {cus} CUs")
+    cases, points, ring_points = [], {}, []
+    for spec in shapes.split(","):
+        k, n = map(int, spec.lower().split("x"))
+        g = torch.Generator(device=dev).manual_seed(k * 31 + n)
+        copies = max(2, -(-ROTATE_BYTES // (k * n)))
+        ws = [torch.randint(-127, 128, (n, k), generator=g, dtype=torch.int8, device=dev)
+              for _ in range(copies)]
+        sb = torch.rand((n, 1), generator=g, device=dev)
+        for m in map(int, ms.split(",")):
+            plan = default_config(m, n, k)
+            c = _lib.CConfig(plan.bm, plan.bn, plan.bk, plan.warps, plan.stages, plan.group_m)
+            _lib.check(_lib.lib().i8l_launch_config(m, n, k, 0, c), RuntimeError)
+            picked = Config(c.bm, c.bn, c.bk, c.warps, c.stages, c.group_m)
+            tiles = (MODEL_MACRO if m > 32 else []) + \
+                (MODEL_DECODE if 16 < m <= 128 else MODEL_SIXTEEN if m <= 16 else [])
+            cands = {Config(t[0], t[1], 128, *t[2:5]): t for t in tiles}
+            cands = {c: t for c, t in cands.items() if supported(m, n, k, c)}
+            if 16 < m <= 128:
+                for z in range(1, 9):
+                    c = Config(max(32, -(-m // 16) * 16), 64, 128, 8, SHARED_RING, z)
+                    if n // 64 * z <= 1024 and supported(m, n, k, c):
+                        cands[c] = None
+            a = torch.randint(-127, 128, (m, k), generator=g, dtype=torch.int8, device=dev)
+            sa = torch.rand((m, 1), generator=g, device=dev)
+            us = {c: time_cold_us(lambda i, c=c: w8a8_mm(a, ws[i % copies].t(), sa, sb,
+                                                         torch.bfloat16, config=c), copies)
+                  for c in dict.fromkeys([plan, picked, *cands])}
+            for c, t in cands.items():
+                if t is None:
+                    ring_points.append((k, n, m, us[c], c.bm, c.group_m))
+                elif m > 128 or t not in MODEL_MACRO:
+                    points.setdefault(t, []).append((k, n, m, us[c]))
+            best = min(us, key=us.get)
+            log(f"K={k} N={n} M={m}: plan {plan.name} {us[plan]:.2f} us, launched {picked.name} "
+                f"{us[picked]:.2f}, fastest {best.name} {us[best]:.2f}")
+            cases.append((k, n, m, us[plan], us[picked], us[best]))
+        del ws
+        torch.cuda.empty_cache()
+
+    def mean(pairs):
+        return round(math.exp(sum(math.log(x / y) for x, y in pairs) / len(pairs)), 4)
+
+    out = {"cases": len(cases), "plan_vs_fastest": mean([(p, b) for *_, p, _, b in cases]),
+           "launched_vs_fastest": mean([(l, b) for *_, _, l, b in cases]),
+           "launched_slower_than_plan": [[k, n, m, round(p, 2), round(l, 2)]
+                                         for k, n, m, p, l, _ in cases if l > 1.02 * p]}
+    log(f"{out}")
+    out["fit"] = {f"{t[0]}x{t[1]} w{t[2]} s{t[3]} g{t[4]}": fit_tile(t, p, cus)
+                  for t, p in points.items() if len(p) >= 6}
+    if len(ring_points) >= 12:
+        out["fit"]["shared ring"] = fit_shared_ring(ring_points, cus)
+    for name, f in out["fit"].items():
+        log(f"{name}: {f}")
+    return out
+
+
 def main() -> int:
     from int8_linear.shapes import SHAPES
     ap = argparse.ArgumentParser()
     ap.add_argument("--ring-costs", action="store_true",
                     help="time the default rule's overlapped-ring tiles (--kn: K x N shapes, "
                          "--m: token counts; defaults: 15 shapes at 48-4096 tokens)")
+    ap.add_argument("--launch-rule", action="store_true",
+                    help="time the tiles i8l_launch_config chooses among, the plan and its pick "
+                         "(--kn: K x N shapes, --m: token counts), and fit its constants")
     ap.add_argument("--shapes", default="qwen3-1.7b-vllm")
     ap.add_argument("--m", default="1,2,4,8,16,17,32,64,128",
                     help="comma-separated M values, or capture (vLLM graph batch sizes)")
@@ -400,6 +541,15 @@ def main() -> int:
         res = ring_costs(args.kn or RING_SHAPES,
                          RING_MS if args.m == ap.get_default("m") else args.m,
                          log=lambda *a: print(*a, file=sys.stderr, flush=True))
+        print(json.dumps(res))
+        return 0
+    if args.launch_rule:
+        res = launch_rule(args.kn or RULE_SHAPES,
+                          RULE_MS if args.m == ap.get_default("m") else args.m,
+                          log=lambda *a: print(*a, file=sys.stderr, flush=True))
+        if args.out:
+            with open(args.out, "w") as f:
+                json.dump(res, f, indent=1)
         print(json.dumps(res))
         return 0
     dev = torch.device("cuda:0")

@@ -575,3 +575,21 @@ def test_launch_config_takes_every_planned_shape():
     assert launched(96, 4096, 6144, split, 1) == split
     for plan in (ring, Config(256, 256, 128, 8, 10, 4), default_config(777, 6144, 4096)):
         assert launched(777, 6144, 4096, plan, 1) == Config(128, 192, 128, 4, 9, 8)
+
+
+@pytest.mark.parametrize("m,k,n,config", [
+    # short K, where the plan's tile of few K steps is the fastest
+    (300, 512, 512, (64, 64, 128, 4, 12, 8)), (400, 384, 768, (64, 64, 128, 4, 12, 8)),
+    (400, 1024, 4096, (128, 64, 128, 4, 12, 8)), (2048, 256, 4096, (256, 128, 128, 8, 11, 8)),
+    # streaming in one round of workgroups; two rounds; more steps a wave; more tokens
+    (33, 1792, 4096, (64, 16, 256, 4, 1, 1)), (48, 768, 3072, (64, 16, 128, 2, 1, 1)),
+    (17, 2304, 4096, (32, 16, 256, 4, 1, 1)), (23, 2176, 4096, (32, 64, 128, 8, 6, 4)),
+    (33, 1280, 5120, (64, 64, 128, 4, 12, 8)), (65, 768, 3072, (64, 64, 128, 4, 12, 8)),
+    # the plan's 256-byte steps on few columns
+    (100, 6144, 2048, (32, 32, 256, 4, 3, 1)), (128, 5120, 2048, (32, 32, 256, 4, 3, 1)),
+    # long K and macro tiles as ever
+    (100, 13824, 5120, (112, 64, 128, 8, 6, 3)), (1500, 5120, 7680, (256, 192, 128, 4, 9, 4))])
+def test_launch_rule_at_measured_points(m, k, n, config):
+    """What is launched without a tuned entry, where the fastest tile (or one within 3% of it) was
+    measured on the GPU."""
+    assert _launched(m, n, k, default_config(m, n, k), 0) == Config(*config)
