@@ -836,7 +836,8 @@ def traffic_summary(kind: str, fetch_csv: str, write_csv: str, run_json: str) ->
     last stdout line (the configs it ran).  Each counter is scaled by what it reads for the
     run's 256 MiB device copies (the largest copy dispatches); the GEMM dispatches (the
     library's kernels, in order) fall into one group per shape, where the kernel or its grid
-    changes, and each group's mean per dispatch is its launch's traffic."""
+    changes or the output of the shape's check is filled (a persistent kernel has one grid for
+    every shape), and each group's mean per dispatch is its launch's traffic."""
     import csv
 
     def load(path):
@@ -854,6 +855,8 @@ def traffic_summary(kind: str, fetch_csv: str, write_csv: str, run_json: str) ->
         groups, prev = [], None
         for d in ds:
             if "i8l::" not in meta[d][0] or "gemm" not in meta[d][0]:
+                if "FillFunctor" in meta[d][0] and meta[d][1] > 1 << 20:
+                    prev = None   # (torch.equal's and any()'s fills are small)
                 continue
             if meta[d] != prev:
                 groups.append([])

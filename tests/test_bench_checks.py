@@ -204,3 +204,40 @@ def test_traffic_summary_groups_launches_and_scales_by_the_copies(tmp_path):
     assert sh["down_proj"]["fetch_kib_per_launch"] == 170000.0
     m, k, n = 4096, 4096, 6144
     assert sh["qkv_proj"]["algorithmic_bytes_per_launch"] == m * k + k * n + 4 * m + 4 * n + 2 * m * n
+
+
+def test_traffic_summary_tells_a_persistent_kernels_shapes_apart(tmp_path):
+    """One kernel on one grid for every shape (a persistent tile): the groups begin where the output
+    of a shape's check is filled, not at the small fills between the launches of one shape."""
+    import csv as csvmod
+
+    def write(path, col):
+        rows, did = [], 0
+
+        def add(name, grid, val):
+            nonlocal did
+            did += 1
+            rows.append([did, name, grid, col, val])
+
+        for i in range(4):
+            add("at::native::vectorized_elementwise_kernel<FillFunctor<BFloat16>>", 2 << 20, 8.0)
+            add("void i8l::gemm_phased<2, 2>(int)", 65536, 1000.0 * (i + 1))
+            for _ in range(2):
+                add("at::native::vectorized_elementwise_kernel<FillFunctor<bool>>", 256, 1.0)
+                add("void i8l::gemm_phased<2, 2>(int)", 65536, 1000.0 * (i + 1))
+        for _ in range(3):
+            add("__amd_rocclr_copyBuffer", 131072, 131072.0 if col == "FETCH_SIZE" else 262144.0)
+        with open(path, "w", newline="") as fh:
+            wr = csvmod.writer(fh)
+            wr.writerow(["Dispatch_Id", "Kernel_Name", "Grid_Size", "Counter_Name", "Counter_Value"])
+            wr.writerows(rows)
+
+    write(tmp_path / "f.csv", "FETCH_SIZE")
+    write(tmp_path / "w.csv", "WRITE_SIZE")
+    run = {"prefill": {"per_shape": {lbl: {"kernel": "gemm_phased, config 256x256x128 w4 s9 g4 (x)"}
+                                     for lbl in bench.PREFILL_SHAPES}}}
+    (tmp_path / "run.out").write_text(json.dumps(run) + "\n")
+    sh = bench.traffic_summary("prefill", str(tmp_path / "f.csv"), str(tmp_path / "w.csv"),
+                               str(tmp_path / "run.out"))["shapes"]
+    assert [sh[lbl]["fetch_kib_per_launch"] for lbl in bench.PREFILL_SHAPES] == \
+        [1000.0, 2000.0, 3000.0, 4000.0]
