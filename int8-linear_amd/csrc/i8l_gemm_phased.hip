@@ -25,8 +25,9 @@ namespace i8l {
 // steps are the next tile's first two, so they fly during the epilogue, which every wave does
 // alone through its own 4 KiB of LDS.
 //
-// What bounds it: power.  On random operands the clock falls to 1.6 GHz (v_mfma alone reaches
-// 3.45 POP/s at 1.77 GHz); leaving out the barriers gains 1%, the LDS reads 8%, the copies 13%.
+// What bounds it: power.  On random operands the clock falls to 1.5-1.6 GHz at 73-77% MFMA busy
+// (v_mfma alone reaches 3.45 POP/s at 1.77 GHz); in timing copies, leaving out the barriers gains
+// 1%, the LDS reads 8%, the copies 13%.
 // So a wave's tile is as large as its registers allow (128 x 128: 256 accumulators), which reads
 // LDS least per MFMA.  Llama-3-8B at 4096 tokens, us: down_proj 199 (gemm_dmap 256x256x128) ->
 // 181 (8 waves of 128x64) -> 174.5 (4 of 128x128), o_proj 63 -> 57.4 -> 55.4, gate_up 433 -> 380.

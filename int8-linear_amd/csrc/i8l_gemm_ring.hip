@@ -12,10 +12,11 @@ namespace i8l {
 // c ^ (r & 7)).  Wave w multiplies columns 16 (w % 4) .. +15 by every token over half w / 4 of each
 // step; the two halves' sums meet once, at the end.
 //
-// What bounds it is the bytes a CU has in flight: LDS-limited (about 140 KiB) against 2-2.5 us of
-// loaded memory latency.  gemm_wlds_a keeps a ring per wave (one or two steps of it in flight), sums
-// its four waves' K slices through LDS and needs two 64-row blocks past 64 tokens, each copying
-// every weight byte.
+// What bounds it is the bytes a CU has in flight, LDS-limited to about 140 KiB: 516 KB go through a
+// CU in 15.2 us (75 tokens, 14336 -> 4096, 4 parts), so a request takes about 4 us to be used; the
+// waves wait for 51% of their cycles, MFMA busy is 8.5%.  gemm_wlds_a keeps a ring per wave (one or
+// two steps of it in flight), sums its four waves' K slices through LDS and needs two 64-row blocks
+// past 64 tokens, each copying every weight byte.
 template <int MT, int EK>
 __global__ void __launch_bounds__(512)
 gemm_ring(const int8_t* __restrict__ A, int64_t lda, const int8_t* __restrict__ B, int64_t ldb,
